@@ -63,9 +63,12 @@
 //   exact scores for every candidate, lists merged across each wave and
 //   then across the waves.
 //
-// * gate_exact_kernel (fp32, take > 16 or unsupported shapes). One thread
-//   per query, exact float64 scores for every candidate, streaming top-T in
-//   registers.
+// * gate_exact_kernel (take > 16 or head dims without a kernel above). One
+//   thread per query, exact float64 scores for every candidate, streaming
+//   top-T in registers.
+//
+// Calls with few blocks per row, and float32 at head_dim 64 / 128, run
+// gate_f64.hip instead.
 #include "common.h"
 
 #include <mutex>
@@ -1716,6 +1719,8 @@ static int run_gate(const void* q, const void* kbar, int32_t* out, const int32_t
                     size_t ws_bytes, hipStream_t st) {
   if constexpr (Elem<T>::kCode == MOBA_FP32) {
     (void)workspace; (void)ws_bytes;
+    if (gate_f64_takes(q, kbar, g, take, MOBA_FP32))
+      return gate_f64(q, kbar, out, cu, g, take, cur, MOBA_FP32, st);
     return dispatch_exact<T>(q, kbar, out, cu, g, take, cur, nullptr, nullptr, st);
   } else {
   // Block ids travel through LDS as 16 bits in the MFMA kernel.
@@ -1726,6 +1731,8 @@ static int run_gate(const void* q, const void* kbar, int32_t* out, const int32_t
   if (!workspace || ws_bytes < moba_gate_workspace_size(g.rows, g.rows_per_seq, g.h_q) ||
       ws_bytes < ws.bytes)
     return fail(MOBA_ERR_WORKSPACE, "gate workspace too small");
+  if (gate_f64_takes(q, kbar, g, take, Elem<T>::kCode))
+    return gate_f64(q, kbar, out, cu, g, take, cur, Elem<T>::kCode, st);
   unsigned* norm_bits = reinterpret_cast<unsigned*>(ws.kbar_norm);
   hipLaunchKernelGGL(gate_init_kernel, dim3(1), dim3(256), 0, st, norm_bits,
                      g.rows * g.h_kv, ws.counter, ws.fb_count, g.rows * g.h_q * kFbBuckets);

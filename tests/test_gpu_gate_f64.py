@@ -1,0 +1,90 @@
+"""The float64 matrix gate (csrc/gate_f64.hip) at the edges of what it takes.
+
+Calls with few blocks per row (and every float32 call at head_dim 64 / 128)
+run it; the same queries against a kbar padded with further rows (ids no
+query may rank) have more blocks per row and run the approximate kernels
+(16-bit types). Both must give the same ids, and the oracle's.
+"""
+
+import pytest
+import torch
+
+from conftest import oracle_cfg
+from moba import _lib
+from moba.config import MoBAConfig
+from moba.kernels.pooling import pool_blocks
+from oracle import c_oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _gate(q, kbar, cfg, rows, take, cu=None):
+    b, s, h, d = q.shape
+    seqs = b if cu is None else cu.numel() - 1
+    out = torch.full((b, h, s, cfg.slots()), -7, dtype=torch.int32, device=q.device)
+    ws = torch.zeros(int(_lib.load().moba_gate_workspace_size(seqs, rows, h)), dtype=torch.uint8,
+                     device=q.device)
+    _lib.call("moba_gate", _lib.ptr(q), _lib.ptr(kbar), _lib.ptr(out), _lib.ptr(cu), seqs, s, rows,
+              h, kbar.shape[1], d, kbar.shape[2], cfg.block_size, cfg.slots(), take,
+              int(cfg.always_select_current), _lib.DTYPE_CODE[q.dtype], _lib.ptr(ws), ws.numel(),
+              _lib.stream_handle(q.device))
+    return out
+
+
+def _padded(kbar, n):
+    pad = torch.full(kbar.shape[:2] + (n - kbar.shape[2], kbar.shape[3]), 9.0, dtype=kbar.dtype,
+                     device=kbar.device)
+    return torch.cat((kbar, pad), 2).contiguous()
+
+
+# (S, query heads, kv heads, head_dim, block, top_k): one query, one block,
+# a tile of 16 blocks or queries less / exactly / plus one, the last block
+# counts of the rule, list lengths 1, 4, 5, 8, 9 and 16 and slots left over.
+CASES = [(1, 1, 1, 64, 16, 4), (15, 2, 1, 64, 16, 1), (16 * 16 + 1, 2, 2, 64, 16, 2),
+         (17 * 16 - 3, 2, 1, 128, 16, 5), (96 * 16, 2, 2, 64, 16, 6), (64 * 32 - 1, 4, 2, 128, 32, 9),
+         (255 * 16 + 16, 1, 1, 64, 16, 10), (255 * 16 - 5, 2, 1, 128, 16, 17), (3 * 128, 2, 2, 64, 128, 16)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("case", CASES)
+def test_gate_f64_matches_oracle_and_general_path(device, case, dtype):
+    s, hq, hk, d, bs, k = case
+    cfg = MoBAConfig(block_size=bs, top_k=k, dtype=dtype)
+    g = torch.Generator().manual_seed(s + d)
+    q = torch.randn((2, s, hq, d), generator=g).to(dtype).to(device)
+    kk = torch.randn((2, s, hk, d), generator=g) + 3.0 * torch.randn((1, 1, hk, d), generator=g)
+    kbar = pool_blocks(kk.to(dtype).to(device), cfg)
+    n = kbar.shape[2]
+    take = cfg.past_blocks_selected(n)
+    got = _gate(q, kbar, cfg, s, take)
+    ref = c_oracle.gate_select(q.cpu(), kbar.cpu(), oracle_cfg(cfg))
+    assert torch.equal(got.cpu(), ref)
+    if dtype != torch.float32:
+        assert torch.equal(got, _gate(q, _padded(kbar, 300), cfg, s, take))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("kind", ["ties", "inf_nan", "tiny", "huge"])
+def test_gate_f64_special_values_match_general_path(device, kind, dtype):
+    """Ties in every place, inf and NaN (which never rank), scores that
+    round to 0 or overflow: the ids of the approximate kernels, whose
+    unsettled queries are rescored one by one. Without the own block too."""
+    cfg = MoBAConfig(block_size=16, top_k=5, dtype=dtype, always_select_current=kind != "ties")
+    lens = [700, 33, 1, 417]
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32).to(device)
+    g = torch.Generator().manual_seed(5)
+    q = torch.randn((1, sum(lens), 4, 64), generator=g)
+    kbar = torch.randn((len(lens), 2, 44, 64), generator=g)
+    if kind == "ties":
+        q, kbar = q.sign(), (kbar * 0.4).round()
+    elif kind == "inf_nan":
+        kbar[0, 0, 3, 5], kbar[0, 1, 7, 0], kbar[0, 0, 20, 1] = float("inf"), float("nan"), -float("inf")
+        q[0, 300, 1, 2], q[0, 500:, 2, 3] = float("nan"), -float("inf")
+    elif kind == "tiny":
+        q, kbar = q * 1e-5, kbar * 1e-3
+    else:
+        q, kbar = q * 2e3, kbar * 10.0
+    q, kbar = q.to(dtype).to(device), kbar.to(dtype).to(device)
+    take = cfg.past_blocks_selected(44)
+    got = _gate(q, kbar, cfg, max(lens), take, cu)
+    assert torch.equal(got, _gate(q, _padded(kbar, 300), cfg, max(lens), take, cu))
