@@ -654,7 +654,22 @@ __device__ __forceinline__ void gate_tile(
   constexpr int BUF_BYTES = CAP * 64 * 6;
   constexpr int WAVE_BYTES = REC_BYTES > BUF_BYTES ? REC_BYTES : BUF_BYTES;
   __shared__ __attribute__((aligned(16))) unsigned char s_wave[WAVES][WAVE_BYTES];
-  __shared__ __attribute__((aligned(16))) uint16_t s_kb[2][SR * KROW];
+  // kbar stages in pass 1, the candidate buffer (C entries and a spare one
+  // per lane) in the decision. The candidates of 8-group lists fit the
+  // stages' bytes. 16-group lists hold up to 64 scores per lane, and on rows
+  // of some hundred blocks a query of 10 to 16 past blocks has most of them
+  // above theta: the 17 entries the stages hold at head_dim 64 overflowed
+  // and most such queries went to the exact queue, one workgroup each. There
+  // the buffer takes LDS of its own (one workgroup per CU either way): 512K
+  // queries of 512 blocks 3108 -> 580 us (top_k 17, bf16, i.i.d. keys),
+  // 711 -> 485 (12), 512 -> 448 (10); head_dim 128 (24 entries before)
+  // 1009 -> 686 at top_k 17, unchanged below 13.
+  constexpr int STAGE_BYTES = 2 * SR * KROW * 2;
+  constexpr int CB = STAGE_BYTES / (NT * 4) - 1;
+  constexpr int C = M > 12 ? 44 : (CB < 24 ? CB : 24);
+  constexpr int KB_BYTES = STAGE_BYTES > (C + 1) * NT * 4 ? STAGE_BYTES : (C + 1) * NT * 4;
+  __shared__ __attribute__((aligned(16))) uint16_t s_kb_[KB_BYTES / 2];
+  uint16_t (*s_kb)[SR * KROW] = reinterpret_cast<uint16_t (*)[SR * KROW]>(s_kb_);
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -977,7 +992,7 @@ __device__ __forceinline__ void gate_tile(
       // id), their records moved to its own slots 0 .. K - 1; every group
       // left out ranks at or below the largest key that left a list (ev).
       float* mk = reinterpret_cast<float*>(&s_kb[0][0]);  // [WAVES][K + 1][64]
-      static_assert(WAVES * (K + 1) * 64 * 4 <= sizeof(s_kb), "merge area");
+      static_assert(WAVES * (K + 1) * 64 * 4 <= sizeof(s_kb_), "merge area");
 #pragma unroll
       for (int p = 0; p < K; ++p) mk[(wave * (K + 1) + p) * 64 + lane] = gk[p];
       mk[(wave * (K + 1) + K) * 64 + lane] = ev;
@@ -1212,8 +1227,6 @@ __device__ __forceinline__ void gate_tile(
   // truncation (less than 2^(IB - 23) |score|).
   constexpr int IB = SLOT_BITS + (GB == 4 ? 2 : 3);
   constexpr uint32_t IMASK = (1u << IB) - 1u;
-  constexpr int CB = (2 * SR * KROW * 2) / (WAVES * 64 * 4) - 1;
-  constexpr int C = CB < 24 ? CB : 24;
   static_assert(C >= 4, "candidate buffer");
   float* cbuf = reinterpret_cast<float*>(&s_kb[0][0]) + wave * (C + 1) * 64 + lane;
   // The kept groups' keys, stored over the records once these are compacted.
