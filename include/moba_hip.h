@@ -250,7 +250,9 @@ int moba_bwd_delta(const void* out, const void* dout, const float* lse,
  * index_stride are those of moba_csc_build. With its segment list, the
  * segments of a cut column leave float32 dK / dV sums in seg_scratch
  * ([R, Hkv, scratch_cap, 2, bs, D] float32, scratch_cap >= 2 * (seg_cap -
- * nb)), which this call then adds in segment order into dK / dV.
+ * nb)), which this call then adds in segment order into dK / dV. float32
+ * inputs sum in float64: their segments need scratch_cap >= 4 * (seg_cap -
+ * nb) on an 8-byte boundary; with less, columns run whole.
  */
 int moba_bwd(const void* q, const void* k, const void* v, const void* dout,
              const float* lse_delta, const int32_t* col_nnz,

@@ -36,7 +36,8 @@ struct AttnArgs {
   const int32_t* seg_split;   // first segment of every cut column
   const int32_t* seg_counts;  // per (row, kv head): segments, cut columns
   int64_t seg_cap;            // entries per (row, kv head)
-  float* seg_scratch;         // backward: fp32 dK / dV of cut columns' segments
+  float* seg_scratch;         // backward: dK / dV of cut columns' segments, float32 sums
+                              // (float32 inputs: float64 sums, in two slots each)
   int64_t scratch_cap;        // scratch slots per (row, kv head)
   int tile_keys;              // FMA attend: keys staged per tile when a block's K / V
                               // exceed LDS (0: the whole block at once)
@@ -113,6 +114,8 @@ __device__ inline int64_t part_row(const AttnArgs& a, const Column& c, int32_t r
 // Kernel launchers implemented per file; each returns MOBA_ERR_UNSUPPORTED
 // when its fast path does not cover the configuration.
 int attend_mfma(const AttnArgs& a, int dtype, int acc_dtype, int64_t n_cols, hipStream_t st);
+int attend_f32(const AttnArgs& a, int dtype, int acc_dtype, int64_t n_cols, hipStream_t st);
+int bwd_f32(const AttnArgs& a, int dtype, int acc_dtype, int64_t n_cols, hipStream_t st);
 int bwd_mfma(const AttnArgs& a, int dtype, int acc_dtype, int64_t n_cols, hipStream_t st);
 
 }  // namespace moba

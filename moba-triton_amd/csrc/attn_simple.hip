@@ -1,11 +1,12 @@
 // KV-block-major attention, forward and backward, in plain float32 FMA.
 //
 // This file holds the C ABI entry points of the attention stages and the
-// general kernels behind them: every dtype (the float32 path always runs
-// here), head_dim a power of two from 8 to 1024. A block whose keys and
-// values do not fit in LDS at once is staged in tiles of keys, with the
-// same arithmetic in the same order. The bf16 / fp16 MFMA kernels (attn_mfma.hip) take the shapes they
-// cover and report MOBA_ERR_UNSUPPORTED otherwise, which routes here.
+// general kernels behind them: every dtype, head_dim a power of two from 8
+// to 1024. A block whose keys and values do not fit in LDS at once is staged
+// in tiles of keys, with the same arithmetic in the same order. The matrix
+// kernels (attn_mfma.hip for bf16 / fp16, attn_f32.hip for float32) take the
+// shapes they cover and report MOBA_ERR_UNSUPPORTED otherwise, which routes
+// here.
 //
 // Semantics restated:
 //   attend : src/moba/kernels/moba_fwd.py:230-425 -- per column, queries x
@@ -741,6 +742,7 @@ extern "C" int moba_attend(const void* q, const void* k, const void* v,
   st = check_launch("moba_attend (fill)");
   if (st) return st;
   st = attend_mfma(a, dtype, acc_dtype, batch * h_kv, s);
+  if (st == MOBA_ERR_UNSUPPORTED) st = attend_f32(a, dtype, acc_dtype, batch * h_kv, s);
   if (st != MOBA_ERR_UNSUPPORTED) return st;
   a.seg = nullptr;  // the FMA kernels take whole columns
   if (!simple_shape_ok(g))
@@ -886,6 +888,7 @@ extern "C" int moba_bwd(const void* q, const void* k, const void* v, const void*
       return check_launch("moba_bwd (cut columns)");
     });
   }
+  if (st == MOBA_ERR_UNSUPPORTED) st = bwd_f32(a, dtype, acc_dtype, batch * h_kv, s);
   if (st != MOBA_ERR_UNSUPPORTED) return st;
   a.seg = nullptr;  // the FMA kernels take whole columns
   if (head_dim > 1024 || head_dim < 8)

@@ -60,10 +60,11 @@ def bwd_kernel(dout, q, k, v, lse_delta, cfg: MoBAConfig, index: CSCIndex, dk, d
     dev = q.device
     rows = index.col_nnz.shape[0]
     mx = index.max_seqlen if index.cu_seqlens is not None else s
-    # float32 dK / dV sums of the segments of cut columns
+    # float32 dK / dV sums of the segments of cut columns (float32 inputs:
+    # float64 sums, two float32 slots each)
     scratch_cap, scratch = 0, None
     if index.segments is not None and index.seg_cap > index.num_blocks:
-        scratch_cap = 2 * (index.seg_cap - index.num_blocks)
+        scratch_cap = 2 * (index.seg_cap - index.num_blocks) * (q.element_size() // 2)
         scratch = torch.empty(rows * h_kv * scratch_cap * 2 * cfg.block_size * d,
                               device=dev, dtype=torch.float32)
     _lib.call("moba_bwd", _lib.ptr(q), _lib.ptr(k), _lib.ptr(v), _lib.ptr(dout),
