@@ -57,15 +57,22 @@ MAX_SEGMENTS = 8
 
 
 def segment_entries(total_pairs: int) -> int:
-    """Longest column segment one program takes: half of one workgroup
-    slot's share of all (query, slot) pairs (about 1024 programs run at
-    once), at least 2048 -- so only columns that would outlast the other
-    programs are cut (none at S = 512K, the longest few at 64K).
+    """Longest column segment one program takes, so that only columns that
+    would outlast the other programs are cut (none at S = 512K, the longest
+    few at 64K): half of one workgroup slot's share of all (query, slot)
+    pairs (about 1024 programs run at once) where that is 2048 or more. On
+    shorter calls a whole share, down to 512: with 2048 as the floor the
+    longest columns ran alone on a mostly idle chip, while every cut costs
+    the backward a float32 dK / dV round trip of the block. Attend / backward
+    in us with segments of 2048, 1024, 512, 256 entries (block 128, top_k 8,
+    four heads of 64): 2K tokens 36/63, 24/51, 18/41, 18/46; 8K 46/91, 33/67,
+    31/72, 30/79; 16K 55/109, 50/104, 47/110, 54/129; 32K 82/159, 79/163,
+    83/203, 95/253.
     `MOBA_SEGMENT_ENTRIES` overrides it; 0 turns cutting off."""
     env = os.environ.get(ENV_SEGMENT)
     if env is not None:
         return int(env)
-    return max(2048, -(-total_pairs // 1024))
+    return max(512, min(2048, -(-total_pairs // 512)), -(-total_pairs // 1024))
 
 
 def index_stride(index: CSCIndex) -> int:
