@@ -69,7 +69,7 @@ count_or_scatter_kernel(const int32_t* __restrict__ block_idx, const int32_t* __
 }
 
 // Tiled count: tq queries of one (row, query head) per workgroup (a tile,
-// tq 256 or kTileQ), kTileT threads each taking up to
+// tq 64, 256 or kTileQ), kTileT threads each taking up to
 // kTileQ / kTileT of them, counted in an LDS histogram over the blocks the
 // tile can see and written out as one row of the unit count table (below).
 // The LDS histogram keeps the global memory traffic at one row per tile:
@@ -81,13 +81,20 @@ constexpr int kTileT = 256;
 
 // Queries per tile (a *unit* of the deterministic build is one tile of one
 // query head): 1024, or 256 when 1024-query tiles would give fewer than 512
-// units. The scatter walks a unit's entries in one serial chain, so a build
-// with few units waits on that chain (256 units at [1,64K,4,64]); with more
-// units, smaller tiles cost more in count-table traffic (units x columns)
-// than they save (measured: 64K 0.088 -> 0.072 ms, 128K no gain).
-inline int64_t tile_queries(int64_t batch, int64_t h_q, int64_t rows_per_seq) {
+// units, or 64 when 256-query tiles would. The scatter walks a unit's entries
+// in one serial chain, so a build with few units waits on that chain (256
+// units at [1,64K,4,64], 32 at [1,2K,4,64]); with more units, smaller tiles
+// cost more in count-table traffic (units x columns) than they save
+// (measured: 256 against 1024 at 64K 0.088 -> 0.072 ms, 128K no gain).
+// A query's ids count up to the last block its tile of visible_queries()
+// queries sees (256 or 1024, whatever the units are).
+inline int64_t visible_queries(int64_t batch, int64_t h_q, int64_t rows_per_seq) {
   const int64_t units = batch * h_q * ((rows_per_seq + kTileQ - 1) / kTileQ);
   return units < 512 ? 256 : kTileQ;
+}
+inline int64_t tile_queries(int64_t batch, int64_t h_q, int64_t rows_per_seq) {
+  const int64_t tq = visible_queries(batch, h_q, rows_per_seq);
+  return tq == 256 && batch * h_q * ((rows_per_seq + 255) / 256) < 512 ? 64 : tq;
 }
 constexpr int kMaxBins = 16384;
 
@@ -119,7 +126,7 @@ __device__ inline void bin_add(int32_t* bins, int32_t blk, bool active) {
 // window [lo, lo + width), zeros where it sees none; grid (tiles, R * Hq).
 __global__ void __launch_bounds__(kTileT)
 tile_count_kernel(const int32_t* __restrict__ block_idx, const int32_t* __restrict__ cu,
-                  int64_t S, int64_t h_q, int64_t n_blocks, int64_t bs, int slots, int tq,
+                  int64_t S, int64_t h_q, int64_t n_blocks, int64_t bs, int slots, int tq, int tv,
                   int32_t* __restrict__ table, int64_t lo, int64_t width) {
   extern __shared__ int32_t bins[];  // width counters (dynamic LDS)
   const int64_t rh = blockIdx.y;
@@ -134,7 +141,8 @@ tile_count_kernel(const int32_t* __restrict__ block_idx, const int32_t* __restri
     return;
   }
   const int64_t t_end = t0 + tq < sp.len ? t0 + tq : sp.len;  // this tile's queries: [t0, t_end)
-  const int nvis = window_visible((t_end - 1) / bs + 1, n_blocks, lo, width);
+  const int64_t v_end = t0 / tv * tv + tv < sp.len ? t0 / tv * tv + tv : sp.len;
+  const int nvis = window_visible((v_end - 1) / bs + 1, n_blocks, lo, width);
   for (int b = threadIdx.x; b < nvis; b += kTileT) bins[b] = 0;
   __syncthreads();
   // Query i of this thread: t0 + threadIdx.x + kTileT * i (a wave's lanes
@@ -267,6 +275,25 @@ chunk_scan_kernel(int32_t* __restrict__ csum, int32_t* __restrict__ col_nnz, int
 // Only columns of the window [lo, lo + width) are placed (the table holds
 // that window). Dynamic LDS: (cursor, mask) pairs of the window's columns.
 constexpr int kPer = 16;
+// Steps 1 to 3 for one row (or half): the position of this lane's entry,
+// whose query is the row's first plus `bit`, in column blk. cm: (cursor, mask)
+// pairs of the wave; `ok` marks lanes with an entry.
+__device__ inline int32_t place_entry(uint32_t* cm, int32_t blk, bool ok, uint32_t bit) {
+  const uint32_t lower = (1u << bit) - 1u;
+  if (ok)
+    __hip_atomic_fetch_or(&cm[2 * blk + 1], 1u << bit, __ATOMIC_RELAXED,
+                          __HIP_MEMORY_SCOPE_WORKGROUP);
+  uint32_t c = 0, m = 0;
+  if (ok) {
+    c = cm[2 * blk];
+    m = cm[2 * blk + 1];
+  }
+  if (ok && (m & lower) == 0u) {
+    cm[2 * blk] = c + __popc(m);
+    cm[2 * blk + 1] = 0u;
+  }
+  return static_cast<int32_t>(c) + __popc(m & lower);
+}
 // Columns the deterministic build handles (8 bytes of LDS each).
 constexpr int kDetMaxCols = kMaxBins;
 constexpr size_t kDetLdsBytes = 8 * static_cast<size_t>(kDetMaxCols);
@@ -276,7 +303,7 @@ det_scatter_kernel(const int32_t* __restrict__ block_idx, const int32_t* __restr
                    int slots, int64_t cap, const int32_t* __restrict__ table,
                    int32_t* __restrict__ row_indices, int32_t* __restrict__ head_indices,
                    int32_t* __restrict__ slot_of_pair, int64_t istride, bool records,
-                   int tq, int64_t lo, int64_t width) {
+                   int tq, int tv, int64_t lo, int64_t width) {
   extern __shared__ uint32_t cm[];  // (cursor, mask) per column of the window
   const int64_t tile = blockIdx.x;
   const int64_t rh = blockIdx.y;
@@ -289,7 +316,8 @@ det_scatter_kernel(const int32_t* __restrict__ block_idx, const int32_t* __restr
   const int64_t t0 = tile * tq;
   if (t0 >= sp.len) return;
   const int64_t t1 = t0 + tq < sp.len ? t0 + tq : sp.len;
-  const int nvis = window_visible((t1 - 1) / bs + 1, n_blocks, lo, width);
+  const int64_t v_end = t0 / tv * tv + tv < sp.len ? t0 / tv * tv + tv : sp.len;
+  const int nvis = window_visible((v_end - 1) / bs + 1, n_blocks, lo, width);
   if (nvis == 0) return;  // no column of the window is visible here
   const int32_t* trow = table + unit * width;
   const int lane = threadIdx.x;
@@ -341,22 +369,8 @@ det_scatter_kernel(const int32_t* __restrict__ block_idx, const int32_t* __restr
         for (int h = 0; h < halves; ++h) {
           const bool ok = valid && (halves == 1 || (lane >> 5) == h);
           const int32_t qrow = __builtin_amdgcn_readlane(q, h * 32);
-          const uint32_t bit = static_cast<uint32_t>(q - qrow);
-          const uint32_t lower = (1u << bit) - 1u;
-          if (ok)
-            __hip_atomic_fetch_or(&cm[2 * blk + 1], 1u << bit, __ATOMIC_RELAXED,
-                                  __HIP_MEMORY_SCOPE_WORKGROUP);
-          uint32_t c = 0, m = 0;
+          const int32_t pos = place_entry(cm, blk, ok, static_cast<uint32_t>(q - qrow));
           if (ok) {
-            c = cm[2 * blk];
-            m = cm[2 * blk + 1];
-          }
-          if (ok && (m & lower) == 0u) {
-            cm[2 * blk] = c + __popc(m);
-            cm[2 * blk + 1] = 0u;
-          }
-          if (ok) {
-            const int32_t pos = static_cast<int32_t>(c) + __popc(m & lower);
             const int64_t dst = (ibase + pos) * istride;
             if (records) {
               *reinterpret_cast<i32x3*>(row_indices + dst) =
@@ -514,48 +528,143 @@ order_sort_kernel(const int32_t* __restrict__ col_nnz, int32_t* __restrict__ ord
 // hold the numbers of segments and of cut columns. One workgroup per
 // (row, kv head); writes past the capacities are dropped (the caller sizes
 // them from an upper bound, so none happen).
+// The next 1024 ranks of the list: `in` marks threads holding a column, of
+// id `col` with `n` entries. carry_*: segments, scratch slots and cut columns
+// so far.
+__device__ inline void segment_ranks(bool in, int32_t col, int64_t n, int64_t rh, int64_t n_blocks,
+                                     int64_t seg_len, int max_seg, int32_t* __restrict__ seg,
+                                     int32_t* __restrict__ split, int64_t cap, int32_t* wtot,
+                                     int32_t& carry_seg, int32_t& carry_scr, int32_t& carry_split) {
+  const int64_t extra_cap = cap - n_blocks;
+  const int64_t k = (n + seg_len - 1) / seg_len;
+  const int32_t nseg = in ? static_cast<int32_t>(k < 1 ? 1 : (k > max_seg ? max_seg : k)) : 0;
+  const int32_t nscr = nseg > 1 ? nseg : 0;
+  int32_t tot_seg, tot_scr, tot_split;
+  const int32_t first = carry_seg + block_scan_1024(nseg, wtot, tot_seg) - nseg;
+  const int32_t first_scr = carry_scr + block_scan_1024(nscr, wtot, tot_scr) - nscr;
+  for (int32_t j = 0; j < nseg; ++j) {
+    const int64_t at = first + j;
+    if (at < cap) {
+      int32_t* e = seg + (rh * cap + at) * 4;
+      e[0] = col;
+      e[1] = j;
+      e[2] = nseg;
+      e[3] = nscr ? first_scr + j : -1;
+    }
+  }
+  const int32_t nth = block_scan_1024(nscr ? 1 : 0, wtot, tot_split);  // cut columns so far
+  if (nscr && carry_split + nth - 1 < extra_cap)
+    split[rh * extra_cap + carry_split + nth - 1] = first;
+  carry_seg += tot_seg;
+  carry_scr += tot_scr;
+  carry_split += tot_split;
+}
+
+__device__ inline void segment_counts(int64_t rh, int64_t n_blocks, int64_t cap, int32_t segments,
+                                      int32_t cut, int32_t* __restrict__ counts) {
+  const int64_t extra_cap = cap - n_blocks;
+  counts[2 * rh] = segments < cap ? segments : static_cast<int32_t>(cap);
+  counts[2 * rh + 1] = cut < extra_cap ? cut : static_cast<int32_t>(extra_cap);
+}
+
 __global__ void __launch_bounds__(1024)
 seg_build_kernel(const int32_t* __restrict__ col_nnz, const int32_t* __restrict__ order,
                  int64_t n_blocks, int64_t seg_len, int max_seg, int32_t* __restrict__ seg,
                  int32_t* __restrict__ split, int32_t* __restrict__ counts, int64_t cap) {
   __shared__ int32_t wtot[16];
   const int64_t rh = blockIdx.x;
-  const int64_t extra_cap = cap - n_blocks;
-  const int tid = threadIdx.x;
   int32_t carry_seg = 0, carry_scr = 0, carry_split = 0;
   for (int64_t base = 0; base < n_blocks; base += 1024) {
-    const int64_t p = base + tid;
-    int32_t nseg = 0;
-    if (p < n_blocks) {
-      const int64_t n = col_nnz[rh * n_blocks + order[rh * n_blocks + p]];
-      const int64_t k = (n + seg_len - 1) / seg_len;
-      nseg = static_cast<int32_t>(k < 1 ? 1 : (k > max_seg ? max_seg : k));
-    }
-    const int32_t nscr = nseg > 1 ? nseg : 0;
-    int32_t tot_seg, tot_scr, tot_split;
-    const int32_t first = carry_seg + block_scan_1024(nseg, wtot, tot_seg) - nseg;
-    const int32_t first_scr = carry_scr + block_scan_1024(nscr, wtot, tot_scr) - nscr;
-    for (int32_t j = 0; j < nseg; ++j) {
-      const int64_t at = first + j;
-      if (at < cap) {
-        int32_t* e = seg + (rh * cap + at) * 4;
-        e[0] = order[rh * n_blocks + p];
-        e[1] = j;
-        e[2] = nseg;
-        e[3] = nscr ? first_scr + j : -1;
-      }
-    }
-    const int32_t nth = block_scan_1024(nscr ? 1 : 0, wtot, tot_split);  // cut columns so far
-    if (nscr && carry_split + nth - 1 < extra_cap)
-      split[rh * extra_cap + carry_split + nth - 1] = first;
-    carry_seg += tot_seg;
-    carry_scr += tot_scr;
-    carry_split += tot_split;
+    const int64_t p = base + threadIdx.x;
+    const bool in = p < n_blocks;
+    const int32_t col = in ? order[rh * n_blocks + p] : 0;
+    segment_ranks(in, col, in ? col_nnz[rh * n_blocks + col] : 0, rh, n_blocks, seg_len, max_seg, seg,
+                  split, cap, wtot, carry_seg, carry_scr, carry_split);
   }
-  if (tid == 0) {
-    counts[2 * rh] = carry_seg < cap ? carry_seg : static_cast<int32_t>(cap);
-    counts[2 * rh + 1] = carry_split < extra_cap ? carry_split : static_cast<int32_t>(extra_cap);
+  if (threadIdx.x == 0) segment_counts(rh, n_blocks, cap, carry_seg, carry_split, counts);
+}
+
+// ---------------------------------------------------------------------------
+// Everything between the count and the scatter in one launch, for (row, kv
+// head) pairs of few columns and units: the scan over the units (unit_chunk,
+// chunk_scan), col_nnz and col_offsets (scan), the column order and the
+// segment list, with the counts in LDS. One workgroup per pair; thread (part
+// p, column b) sums and rescans every P-th part of the units of column b.
+//
+// Bound by latency: on short calls each of the six kernels it replaces is one
+// launch of a few microseconds with little in it. [1, 2048, 4, 64], 128-key
+// blocks, top_k 8: the build's kernels 33 -> 20 us. kMidUnits bounds the
+// units a thread walks; beyond it the six kernels spread over more of the chip.
+constexpr int64_t kMidCols = 1024;
+constexpr int64_t kMidUnits = 32;
+inline bool mid_takes(int64_t n_blocks, int64_t units) {
+  return n_blocks <= kMidCols && units <= kMidUnits * (kMidCols / n_blocks);
+}
+
+__global__ void __launch_bounds__(1024)
+csc_mid_kernel(int32_t* __restrict__ table, int32_t* __restrict__ col_nnz,
+               int32_t* __restrict__ col_offsets, int32_t* __restrict__ order, int nb, int units,
+               int64_t seg_len, int max_seg, int32_t* __restrict__ seg, int32_t* __restrict__ split,
+               int32_t* __restrict__ counts, int64_t seg_cap) {
+  __shared__ int32_t psum[1024];  // [parts][nb]: sums, then each part's base
+  __shared__ int32_t nnz[1024], by_rank[1024];
+  __shared__ int32_t wtot[16];
+  const int64_t rh = blockIdx.x;
+  const int tid = threadIdx.x;
+  const int parts = 1024 / nb;
+  const int part = tid / nb, b = tid - part * nb;
+  const int per = (units + parts - 1) / parts;
+  const int u0 = part * per;
+  const int u1 = part < parts ? (u0 + per < units ? u0 + per : units) : u0;
+  int32_t* col = table + rh * units * nb + b;
+  int32_t acc = 0;
+#pragma unroll 8
+  for (int u = u0; u < u1; ++u) acc += col[static_cast<int64_t>(u) * nb];
+  if (part < parts) psum[tid] = acc;
+  __syncthreads();
+  int32_t mine = 0;
+  if (tid < nb)
+    for (int p = 0; p < parts; ++p) mine += psum[p * nb + tid];
+  int32_t total;
+  const int32_t off = block_scan_1024(mine, wtot, total) - mine;
+  if (tid < nb) {
+    int32_t run = off;
+    for (int p = 0; p < parts; ++p) {
+      const int32_t v = psum[p * nb + tid];
+      psum[p * nb + tid] = run;
+      run += v;
+    }
+    nnz[tid] = mine;
+    col_nnz[rh * nb + tid] = mine;
+    col_offsets[rh * (nb + 1) + tid] = off;
   }
+  if (tid == 0) col_offsets[rh * (nb + 1) + nb] = total;
+  __syncthreads();
+  int32_t run = part < parts ? psum[tid] : 0;
+#pragma unroll 8
+  for (int u = u0; u < u1; ++u) {
+    const int32_t v = col[static_cast<int64_t>(u) * nb];
+    col[static_cast<int64_t>(u) * nb] = run;
+    run += v;
+  }
+
+  // Longest first, ties by id: each column's rank.
+  if (tid < nb) {
+    int rank = 0;
+    for (int o = 0; o < nb; ++o) {
+      const int32_t n = nnz[o];
+      rank += (n > mine || (n == mine && o < tid)) ? 1 : 0;
+    }
+    order[rh * nb + rank] = tid;
+    by_rank[rank] = tid;
+  }
+  if (!seg) return;  // uniform
+  __syncthreads();
+  const int32_t c = tid < nb ? by_rank[tid] : 0;
+  int32_t n_seg = 0, n_scr = 0, n_cut = 0;
+  segment_ranks(tid < nb, c, nnz[c], rh, nb, seg_len, max_seg, seg, split, seg_cap, wtot, n_seg, n_scr,
+                n_cut);
+  if (tid == 0) segment_counts(rh, nb, seg_cap, n_seg, n_cut, counts);
 }
 
 }  // namespace moba
@@ -658,6 +767,8 @@ extern "C" int moba_csc_build(const int32_t* block_idx, int32_t* col_nnz,
   const int64_t bs_eff = cdiv(g.rows_per_seq, n_blocks);
   const int64_t tq = tile_queries(batch, h_q, g.rows_per_seq);
   const UnitPlan up = unit_plan(g.rows_per_seq, h_q, h_kv, tq);
+  const int tv = static_cast<int>(visible_queries(batch, h_q, g.rows_per_seq));
+  const bool mid = tiled && n_win == 1 && mid_takes(n_blocks, up.units);
   const unsigned rhk = static_cast<unsigned>(batch * h_kv);
   dim3 grid(static_cast<unsigned>(cdiv(g.rows_per_seq * slots, 256)),
             static_cast<unsigned>(batch * h_q));
@@ -671,7 +782,8 @@ extern "C" int moba_csc_build(const int32_t* block_idx, int32_t* col_nnz,
     hipLaunchKernelGGL(tile_count_kernel, tgrid, dim3(kTileT),
                        static_cast<unsigned>(sizeof(int32_t) * width), s, block_idx, cu_seqlens,
                        seq_len, h_q, n_blocks, bs_eff, static_cast<int>(slots),
-                       static_cast<int>(tq), table, lo, width);
+                       static_cast<int>(tq), tv, table, lo, width);
+    if (mid) return;
     hipLaunchKernelGGL(unit_chunk_kernel<0>,
                        dim3(static_cast<unsigned>(cdiv(width, 256)),
                             static_cast<unsigned>(up.nchunks), rhk),
@@ -681,16 +793,17 @@ extern "C" int moba_csc_build(const int32_t* block_idx, int32_t* col_nnz,
                        dim3(256), 0, s, csum, nnz, n_blocks, up.nchunks, width);
   };
   auto window_place = [&](int64_t lo, int64_t width) {
-    hipLaunchKernelGGL(unit_chunk_kernel<1>,
-                       dim3(static_cast<unsigned>(cdiv(width, 256)),
-                            static_cast<unsigned>(up.nchunks), rhk),
-                       dim3(256), 0, s, table, csum, col_offsets, n_blocks, h_q, h_kv,
-                       up.units, up.chunk, up.nchunks, lo, width);
+    if (!mid)
+      hipLaunchKernelGGL(unit_chunk_kernel<1>,
+                         dim3(static_cast<unsigned>(cdiv(width, 256)),
+                              static_cast<unsigned>(up.nchunks), rhk),
+                         dim3(256), 0, s, table, csum, col_offsets, n_blocks, h_q, h_kv,
+                         up.units, up.chunk, up.nchunks, lo, width);
     hipLaunchKernelGGL(det_scatter_kernel, tgrid, dim3(64),
                        static_cast<unsigned>(8 * width), s, block_idx, cu_seqlens, seq_len, h_q,
                        h_kv, n_blocks, bs_eff, static_cast<int>(slots), cap, table, row_indices,
                        head_indices, slot_of_pair, index_stride, records, static_cast<int>(tq),
-                       lo, width);
+                       tv, lo, width);
   };
   if (tiled && n_win == 1) {
     window_counts(0, n_blocks, col_nnz);
@@ -703,6 +816,13 @@ extern "C" int moba_csc_build(const int32_t* block_idx, int32_t* col_nnz,
                        cu_seqlens, seq_len, g.rows_per_seq, h_q, h_kv, n_blocks,
                        static_cast<int>(slots), cap, col_nnz, nullptr, nullptr, nullptr,
                        nullptr, index_stride);
+  }
+  if (mid) {
+    hipLaunchKernelGGL(csc_mid_kernel, dim3(rhk), dim3(1024), 0, s, table, col_nnz, col_offsets, order,
+                       static_cast<int>(n_blocks), static_cast<int>(up.units), seg_len,
+                       static_cast<int>(max_seg), segments, seg_split, seg_counts, seg_cap);
+    window_place(0, n_blocks);
+    return check_launch("moba_csc_build");
   }
   hipLaunchKernelGGL(scan_kernel, dim3(rhk), dim3(1024), 0, s, col_nnz, col_offsets, n_blocks);
   int n2 = 1;
