@@ -468,7 +468,7 @@ bwd_f32_kernel(AttnArgs a) {
 }
 
 // dK / dV of the cut columns: the segments' float64 sums added in segment
-// order and rounded once. One workgroup per cut column.
+// order and rounded once. Eight workgroups per cut column.
 __global__ void __launch_bounds__(256) seg_finish_f32_kernel(AttnArgs a) {
   const int64_t rh = blockIdx.y;
   if (static_cast<int64_t>(blockIdx.x) >= a.seg_counts[2 * rh + 1]) return;
@@ -477,7 +477,7 @@ __global__ void __launch_bounds__(256) seg_finish_f32_kernel(AttnArgs a) {
   const double* base = reinterpret_cast<const double*>(a.seg_scratch) +
                        (rh * (a.scratch_cap / 2) + c.scratch) * 2 * bsd;
   const int64_t n = (c.key_end - c.key0) * a.D;
-  for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
+  for (int64_t i = blockIdx.z * blockDim.x + threadIdx.x; i < n; i += gridDim.z * blockDim.x) {
     double sk = 0.0, sv = 0.0;
     for (int j = 0; j < c.nseg; ++j) {
       sk += base[j * 2 * bsd + i];
@@ -519,7 +519,7 @@ int launch_bwd(const AttnArgs& args, int64_t n_cols, hipStream_t st) {
   const int rc = check_launch("moba_bwd (float32)");
   if (rc || !a.seg || a.seg_cap == a.n_blocks) return rc;
   hipLaunchKernelGGL(seg_finish_f32_kernel,
-                     dim3(static_cast<unsigned>(a.seg_cap - a.n_blocks), static_cast<unsigned>(n_cols)),
+                     dim3(static_cast<unsigned>(a.seg_cap - a.n_blocks), static_cast<unsigned>(n_cols), 8),
                      dim3(256), 0, st, a);
   return check_launch("moba_bwd (float32, cut columns)");
 }
