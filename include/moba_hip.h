@@ -170,7 +170,8 @@ int moba_gate_noalloc(const void* q, const void* kbar, int32_t* block_idx,
  */
 /* Workspace of moba_csc_build in bytes; rows_per_seq is seq_len, or
  * max_seqlen when packed. With W = min(nb, 16384) it holds a count table of
- * R * Hq * ceil(rows_per_seq / 1024) * W int32 plus chunk sums of
+ * R * Hq * ceil(rows_per_seq / tile) * W int32 (tiles of 1024 queries, 256
+ * or 64 on shorter calls) plus chunk sums of
  * R * Hkv * W * (at most 64) int32 (never less than R * Hkv * nb int32, the
  * atomic cursors of the fallback). */
 size_t moba_csc_workspace_size(int64_t batch, int64_t rows_per_seq, int64_t h_q,
@@ -278,6 +279,41 @@ int moba_dq_reduce(const void* dq_part, const float* part_m, int64_t m_stride, v
                    int64_t batch, int64_t seq_len, int64_t h_q,
                    int64_t head_dim, int64_t slots, int acc_dtype,
                    int out_dtype, void* stream);
+
+/*
+ * A whole forward (pool, gate, CSC build, attend, merge) or backward (delta,
+ * backward, dQ reduce) in one call: the stages above in order on one stream,
+ * with their buffers carved from two the caller allocates. On short
+ * sequences a caller's own per-stage work (allocations, argument lists) is
+ * most of a step's time.
+ *
+ * Fill every field of the first group, call moba_step_layout for n_blocks and
+ * the sizes, allocate, fill the pointers, run. `saved` holds what the
+ * backward reads (CSC index, segment list, (m, l) pairs, lse) and is kept
+ * until then; `temp` (forward_temp / backward_temp bytes) is free again when
+ * the stage's work on the stream is done. With keep = 0 (no backward will
+ * follow) `saved` may be freed likewise, and no lse is formed. All buffers on
+ * 256-byte boundaries. Partials are in the input dtype. On failure
+ * failed_stage names the stage: 1 pool, 2 gate, 3 csc_build, 4 attend, 5
+ * combine, 6 bwd_delta, 7 bwd, 8 dq_reduce (0: the call's own checks).
+ */
+typedef struct moba_step {
+  /* shape and configuration; batch, seq_len, max_seqlen as in every call */
+  int64_t batch, seq_len, max_seqlen, h_q, h_kv, head_dim, block_size, slots, take;
+  int64_t always_current, causal, dtype, dkv_dtype, keep, packed;
+  int64_t seg_len, max_seg; /* seg_len 0: no segment list */
+  /* set by moba_step_layout */
+  int64_t n_blocks, saved_bytes, forward_temp, backward_temp, failed_stage;
+  /* device pointers */
+  const void *q, *k, *v;
+  const int32_t* cu_seqlens;
+  void *out, *saved, *temp;
+  const void* dout; /* backward only, as dq / dk / dv */
+  void *dq, *dk, *dv;
+} moba_step;
+int moba_step_layout(moba_step* step);
+int moba_forward_step(moba_step* step, void* stream);
+int moba_backward_step(moba_step* step, void* stream);
 
 #ifdef __cplusplus
 }

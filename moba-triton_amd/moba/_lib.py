@@ -50,7 +50,26 @@ SIGNATURES = {
                       _L, _L, _L, _L, _L, _L, _L, _L, _L, _L, _L, _P, _P, _P, _L, _P, _L,
                       _I, _I, _I, _I, _P]),
     "moba_dq_reduce": (_I, [_P, _P, _L, _P, _L, _L, _L, _L, _L, _I, _I, _P]),
+    "moba_step_layout": (_I, [_P]),
+    "moba_forward_step": (_I, [_P, _P]),
+    "moba_backward_step": (_I, [_P, _P]),
 }
+
+
+class Step(ctypes.Structure):
+    """`moba_step` of include/moba_hip.h."""
+
+    _fields_ = ([(n, _L) for n in (
+        "batch", "seq_len", "max_seqlen", "h_q", "h_kv", "head_dim", "block_size", "slots", "take",
+        "always_current", "causal", "dtype", "dkv_dtype", "keep", "packed", "seg_len", "max_seg",
+        "n_blocks", "saved_bytes", "forward_temp", "backward_temp", "failed_stage")] +
+        [(n, _P) for n in ("q", "k", "v", "cu_seqlens", "out", "saved", "temp", "dout", "dq", "dk",
+                           "dv")])
+
+
+# Entry point behind each value of Step.failed_stage.
+_STAGES = (None, "moba_pool", "moba_gate", "moba_csc_build", "moba_attend", "moba_combine",
+           "moba_bwd_delta", "moba_bwd", "moba_dq_reduce")
 
 _lib = None
 
@@ -116,8 +135,20 @@ def call(name: str, *args) -> None:
     RuntimeError."""
     lib = load()
     rc = getattr(lib, name)(*args)
-    if rc == MOBA_OK:
-        return
+    if rc != MOBA_OK:
+        _raise(lib, name, rc)
+
+
+def run_step(name: str, step: Step, *stream) -> None:
+    """As `call`, for the entry points on a `Step`; an error names the stage
+    that failed."""
+    lib = load()
+    rc = getattr(lib, name)(ctypes.byref(step), *stream)
+    if rc != MOBA_OK:
+        _raise(lib, _STAGES[step.failed_stage] or name, rc)
+
+
+def _raise(lib, name: str, rc: int) -> None:
     msg = lib.moba_last_error().decode(errors="replace")
     if rc in (MOBA_ERR_INVALID, MOBA_ERR_UNSUPPORTED):
         raise ValueError(f"{name}: {msg}")

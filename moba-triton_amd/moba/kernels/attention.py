@@ -2,8 +2,9 @@
 (reference `src/moba/kernels/attention.py`).
 
 Saved for backward: q, k, v, out and, per chunk, lse (log2 units), part_m
-(the written-marker of the per-slot partials) and the CSC index. The gate
-receives no gradient (`attention.py:33-38`): routing is a hard top-k.
+(the written-marker of the per-slot partials) and the CSC index -- in one
+buffer (`step.SavedStep`) unless the caller gave the index. The gate receives
+no gradient (`attention.py:33-38`): routing is a hard top-k.
 """
 
 import torch
@@ -14,6 +15,8 @@ from moba.config import MoBAConfig
 from moba.kernels.moba_bwd import moba_backward
 from moba.kernels.moba_fwd import _validate, attend_partials, combine_partials
 from moba.kernels.routing import CSCIndex, build_csc_fused
+from moba.kernels.step import SavedStep
+from moba.kernels import step
 
 
 def _piece(t, b0, b1, h0, h1):
@@ -67,29 +70,38 @@ class MoBAAttentionFunction(torch.autograd.Function):
             qc = q if whole else _piece(q, b0, b1, hq0, hq1)
             kc = k if whole else _piece(k, b0, b1, hk0, hk1)
             vc = v if whole else _piece(v, b0, b1, hk0, hk1)
-            idx = index if index is not None else build_csc_fused(
-                qc, kc, cfg, cu_seqlens=cu_seqlens, max_seqlen=max_seqlen)
-            part_m, part_l, part_acc = attend_partials(qc, kc, vc, cfg, idx, causal=causal)
-            oc, lse = combine_partials(part_m, part_l, part_acc, q.dtype, return_lse=True)
-            del part_l, part_acc
+            if index is None and cfg.gate_group == 0:
+                oc, kept = step.forward(qc, kc, vc, cfg, causal, cu_seqlens, max_seqlen, keep=True)
+            else:
+                idx = index if index is not None else build_csc_fused(
+                    qc, kc, cfg, cu_seqlens=cu_seqlens, max_seqlen=max_seqlen)
+                part_m, part_l, part_acc = attend_partials(qc, kc, vc, cfg, idx, causal=causal)
+                oc, lse = combine_partials(part_m, part_l, part_acc, q.dtype, return_lse=True)
+                del part_l, part_acc
+                kept = (idx, lse, part_m)
             if whole:
                 out = oc
             else:
                 out[b0:b1, :, hq0:hq1] = oc
-            saved.append((idx, lse, part_m))
+            saved.append(kept)
         ctx.save_for_backward(q, k, v, out)
         ctx.cfg, ctx.causal, ctx.chunks, ctx.saved = cfg, causal, chunks, saved
-        ctx.index = saved[0][0] if len(chunks) == 1 else None
         return out
+
+    @staticmethod
+    def _chunk_backward(ctx, kept, dout, q, k, v, out, dkv_dtype=None):
+        if isinstance(kept, SavedStep):
+            return step.backward(dout, q, k, v, out, kept, dkv_dtype)
+        idx, lse, part_m = kept
+        return moba_backward(dout, q, k, v, out, lse, part_m, ctx.cfg, idx, causal=ctx.causal,
+                             dkv_dtype=dkv_dtype)
 
     @staticmethod
     def backward(ctx, dout):
         q, k, v, out = ctx.saved_tensors
         chunks, group = ctx.chunks, q.shape[2] // k.shape[2]
         if len(chunks) == 1:
-            idx, lse, part_m = ctx.saved[0]
-            dq, dk, dv = moba_backward(dout, q, k, v, out, lse, part_m, ctx.cfg, idx,
-                                       causal=ctx.causal)
+            dq, dk, dv = MoBAAttentionFunction._chunk_backward(ctx, ctx.saved[0], dout, q, k, v, out)
             return dq, dk, dv, None, None, None, None, None
         # Chunks holding part of a kv head's group add their unrounded
         # float32 dK / dV; the sum is rounded once.
@@ -98,13 +110,13 @@ class MoBAAttentionFunction(torch.autograd.Function):
         dk, dv = ((torch.zeros(k.shape, dtype=torch.float32, device=k.device),
                    torch.zeros(v.shape, dtype=torch.float32, device=v.device)) if split
                   else (torch.empty_like(k), torch.empty_like(v)))
-        for chunk, (idx, lse, part_m) in zip(chunks, ctx.saved):
+        for chunk, kept in zip(chunks, ctx.saved):
             b0, b1, hk0, hk1 = chunk[:4]
             hq0, hq1 = query_heads(chunk, group)
-            g = moba_backward(_piece(dout, b0, b1, hq0, hq1), _piece(q, b0, b1, hq0, hq1),
-                              _piece(k, b0, b1, hk0, hk1), _piece(v, b0, b1, hk0, hk1),
-                              _piece(out, b0, b1, hq0, hq1), lse, part_m, ctx.cfg, idx,
-                              causal=ctx.causal, dkv_dtype=torch.float32 if split else None)
+            g = MoBAAttentionFunction._chunk_backward(
+                ctx, kept, _piece(dout, b0, b1, hq0, hq1), _piece(q, b0, b1, hq0, hq1),
+                _piece(k, b0, b1, hk0, hk1), _piece(v, b0, b1, hk0, hk1),
+                _piece(out, b0, b1, hq0, hq1), torch.float32 if split else None)
             dq[b0:b1, :, hq0:hq1] = g[0]
             if split:
                 dk[b0:b1, :, hk0:hk1] += g[1]

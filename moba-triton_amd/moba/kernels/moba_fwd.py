@@ -205,6 +205,7 @@ def moba_forward(q, k, v, cfg: MoBAConfig, index: CSCIndex | None = None,
     # Without a caller's index the per-slot buffers are bounded by running
     # (batch row, kv head[, query heads]) chunks (moba.chunking).
     from moba.chunking import query_heads
+    from moba.kernels import step
     from moba.kernels.attention import _piece, forward_chunks
     chunks = forward_chunks(q, k, v, cfg, causal, cu_seqlens, max_seqlen,
                             partials_dtype=partials_dtype)
@@ -217,10 +218,13 @@ def moba_forward(q, k, v, cfg: MoBAConfig, index: CSCIndex | None = None,
         qc = q if whole else _piece(q, b0, b1, hq0, hq1)
         kc = k if whole else _piece(k, b0, b1, hk0, hk1)
         vc = v if whole else _piece(v, b0, b1, hk0, hk1)
-        idx = build_csc_fused(qc, kc, cfg, cu_seqlens=cu_seqlens, max_seqlen=max_seqlen)
-        part_m, part_l, part_acc = attend_partials(qc, kc, vc, cfg, idx, causal=causal,
-                                                   partials_dtype=partials_dtype)
-        oc = combine_partials(part_m, part_l, part_acc, q.dtype)
+        if partials_dtype is None and cfg.gate_group == 0:
+            oc, _ = step.forward(qc, kc, vc, cfg, causal, cu_seqlens, max_seqlen, keep=False)
+        else:
+            idx = build_csc_fused(qc, kc, cfg, cu_seqlens=cu_seqlens, max_seqlen=max_seqlen)
+            part_m, part_l, part_acc = attend_partials(qc, kc, vc, cfg, idx, causal=causal,
+                                                       partials_dtype=partials_dtype)
+            oc = combine_partials(part_m, part_l, part_acc, q.dtype)
         if whole:
             return oc
         out[b0:b1, :, hq0:hq1] = oc

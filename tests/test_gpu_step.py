@@ -1,0 +1,59 @@
+"""The whole-step entry points (csrc/step.cpp) against the stages called one by
+one: with the same index, output and gradients are the same bits.
+"""
+
+import pytest
+import torch
+
+from conftest import make_qkv
+from moba.config import MoBAConfig
+from moba.kernels.attention import moba_attention
+from moba.kernels.moba_fwd import moba_forward
+from moba.kernels.routing import build_csc_fused
+
+pytestmark = pytest.mark.gpu
+
+# (S or packed lengths, batch, query heads, kv heads, head_dim, block, top_k, dtype)
+CASES = [(515, 2, 4, 2, 64, 64, 4, torch.bfloat16), (1, 1, 2, 2, 64, 32, 8, torch.float16),
+         ([130, 1, 700], 1, 8, 2, 128, 64, 3, torch.bfloat16), (400, 1, 4, 1, 64, 32, 1, torch.float32),
+         ([64, 900], 1, 4, 4, 64, 128, 6, torch.float32), (300, 1, 2, 1, 256, 32, 3, torch.bfloat16)]
+
+
+@pytest.mark.parametrize("entries", ["0", "64", None])
+@pytest.mark.parametrize("case", CASES)
+def test_step_equals_stages(device, monkeypatch, case, entries):
+    """No segment list, cut columns, the default; a backward run twice."""
+    if entries is not None:
+        monkeypatch.setenv("MOBA_SEGMENT_ENTRIES", entries)
+    s, b, hq, hk, d, bs, k, dtype = case
+    lens = s if isinstance(s, list) else None
+    t = sum(lens) if lens else s
+    cfg = MoBAConfig(block_size=bs, top_k=k, dtype=dtype)
+    q, do = make_qkv((b, t, hq, d), dtype, seed=1, device=device, n=2)
+    kk, v = make_qkv((b, t, hk, d), dtype, seed=2, device=device, n=2)
+    kw = {}
+    if lens:
+        kw = {"cu_seqlens": torch.tensor([0] + lens).cumsum(0).to(torch.int32).to(device),
+              "max_seqlen": max(lens)}
+    index = build_csc_fused(q, kk, cfg, **kw)
+    results = []
+    for given in (index, None):
+        x = [z.clone().requires_grad_(True) for z in (q, kk, v)]
+        out = moba_attention(*x, cfg, index=given, **({} if given is not None else kw))
+        grads = torch.autograd.grad(out, x, do, retain_graph=True)
+        again = torch.autograd.grad(out, x, do)
+        assert all(torch.equal(a, c) for a, c in zip(grads, again))
+        results.append((out.detach(), *grads))
+    assert all(torch.equal(a, c) for a, c in zip(*results))
+    assert torch.equal(moba_forward(q, kk, v, cfg, **kw), results[0][0])
+    assert torch.equal(moba_forward(q, kk, v, cfg, index=index), results[0][0])
+
+
+def test_step_errors_name_the_stage(device):
+    """A shape a stage refuses (the gate takes at most 128 past blocks) fails
+    with that stage's message, as the stage called alone."""
+    cfg = MoBAConfig(block_size=16, top_k=200, dtype=torch.float32)
+    q, k, v = make_qkv((1, 4096, 1, 64), torch.float32, device=device)
+    for call in (lambda: build_csc_fused(q, k, cfg), lambda: moba_forward(q, k, v, cfg)):
+        with pytest.raises(ValueError, match="moba_gate: gate supports at most 128"):
+            call()
