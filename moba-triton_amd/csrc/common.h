@@ -82,7 +82,14 @@ template <> struct Elem<bf16_t> {
 };
 template <> struct Elem<f16_t> {
   static constexpr int kCode = MOBA_FP16;
-  __device__ static float load(const f16_t* p, int64_t i) { return f16_to_float(p[i].bits); }
+  // By the hardware conversion (v_cvt_f32_f16; exact, subnormals included:
+  // the library is built with the default float16 denormal mode, which keeps
+  // them). The integer form above takes a dozen instructions per element,
+  // which set the time of the passes over partial rows: merging 2.1M rows of
+  // 8 slots, D 64, took 822 us against 453 in bf16.
+  __device__ static float load(const f16_t* p, int64_t i) {
+    return static_cast<float>(__builtin_bit_cast(_Float16, p[i].bits));
+  }
   __device__ static void store(f16_t* p, int64_t i, float v) { p[i].bits = float_to_f16(v); }
   __device__ static float round(float v) { return f16_to_float(float_to_f16(v)); }
 };
