@@ -407,8 +407,8 @@ int attend_mfma(const AttnArgs& a, int dtype, int acc_dtype, int64_t n_cols, hip
 }
 
 // ---------------------------------------------------------------------------
-// Backward (bwd_mfma_kernel): one workgroup per (KV block, row * kv head),
-// one wave per 32 keys of the block. The workgroup owns its keys' dK / dV
+// Backward, head_dim 64 (bwd_mfma_kernel): one workgroup per (KV block, row *
+// kv head), one wave per 32 keys of the block. The workgroup owns its keys' dK / dV
 // for the whole column (registers, stored once: no atomics), and walks the
 // column in steps of 64 entries. Per step, with the step's Q / dO rows
 // staged in LDS (row-major; the transposed operands come from transposing
@@ -425,7 +425,7 @@ int attend_mfma(const AttnArgs& a, int dtype, int acc_dtype, int64_t n_cols, hip
 // inside the workgroup, so the partial buffer is [.., slots, D], not
 // slots x sub-tiles. Semantics: src/moba/kernels/moba_bwd.py:216-394.
 // ---------------------------------------------------------------------------
-// Piece permutation of a Q / dO tile row (bwd_mfma_kernel at head_dim 64):
+// Piece permutation of a Q / dO tile row (bwd_mfma_kernel):
 // bits 1-3 of the row, reversed. Rows 2i and 2i + 1 share it; the eight
 // even (odd) rows of 16 consecutive ones take eight distinct values, and
 // rows 4a, 4a + 1 and 4a + 2, 4a + 3 differ in bit 2, which moves a
@@ -434,61 +434,80 @@ __device__ constexpr int bq_swz(int row) {
   return (((row >> 1) & 1) << 2) | ((row >> 1) & 2) | ((row >> 3) & 1);
 }
 
-template <typename T, typename A, int D, int BS, int NQ, int ST>
-__global__ void __launch_bounds__(BS * 2 * ST, (D == 64 && BS == 128) ? 2 : 1)
+// dK, dV of this lane's key: register v of tile dt is feature f0 + 32dt +
+// 8(v/4) + v%4. A segment of a cut column leaves its float32 sums in its
+// scratch slot ([2][BS][D]: dK scaled, dV); the finishing pass adds the
+// column's segments in order.
+template <typename T, int D, int BS, int DT>
+__device__ inline void store_dkv(const AttnArgs& a, const Column& c, int key, int key_lim, int f0,
+                                 const floatx16_t (&dk)[DT], const floatx16_t (&dv)[DT]) {
+  if (key >= key_lim) return;
+  auto store = [&](auto* dK, auto* dV) {
+    using E = std::remove_pointer_t<decltype(dK)>;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int q4 = 0; q4 < 4; ++q4) {
+        store4<E>(dK + dt * 32 + 8 * q4, dk[dt][4 * q4] * a.scale, dk[dt][4 * q4 + 1] * a.scale,
+                  dk[dt][4 * q4 + 2] * a.scale, dk[dt][4 * q4 + 3] * a.scale);
+        store4<E>(dV + dt * 32 + 8 * q4, dv[dt][4 * q4], dv[dt][4 * q4 + 1],
+                  dv[dt][4 * q4 + 2], dv[dt][4 * q4 + 3]);
+      }
+  };
+  if (c.nseg > 1) {
+    float* sk = a.seg_scratch +
+                (static_cast<int64_t>(blockIdx.y) * a.scratch_cap + c.scratch) * 2 * BS * D +
+                key * D + f0;
+    store(sk, sk + BS * D);
+    return;
+  }
+  const int64_t off = ((c.tok0 + key) * a.h_kv + c.hk) * D + f0;
+  if (a.dkv_f32)  // uniform: float32 sums for a caller that adds several calls
+    store(static_cast<float*>(a.dk) + off, static_cast<float*>(a.dv) + off);
+  else
+    store(static_cast<T*>(a.dk) + off, static_cast<T*>(a.dv) + off);
+}
+
+template <typename T, typename A, int BS>
+__global__ void __launch_bounds__(BS * 2, BS == 128 ? 2 : 1)
 bwd_mfma_kernel(AttnArgs a) {
   using M = Mfma<T>;
   using V8 = typename M::vec;
   using Sc = typename M::scalar;
-  // NQ: queries per step (64; 32 at head_dim 128 with blocks under 128 keys)
+  constexpr int D = 64;
+  constexpr int NQ = 64;        // queries per step
   constexpr int QT = NQ / 32;   // query tiles of 32
-  constexpr int NW = BS / 32;   // waves per stream: 32 keys each
-  constexpr int NT = NW * 64;   // threads per stream
-  constexpr int NTA = NT * ST;  // threads
-  // ST = 2: two streams of waves walk alternate steps of the column against
-  // the same keys, each with its own rows, dS^T and dK / dV sums (added at
-  // the end). K and V then sit row-major in LDS instead of in each lane's
-  // registers (S / dP read their B operands from there, dQ its K^T operand
-  // by transposing reads), which keeps a wave within 256 registers so a CU
-  // runs two of them per SIMD.
-  constexpr bool kKV = ST > 1;
+  constexpr int NW = BS / 32;   // waves: 32 keys each
+  constexpr int NT = NW * 64;   // threads
   constexpr int DT = D / 32;
-  constexpr int RS = D + 8;     // row stride of [key|q][d] tiles
-  // Q / dO tiles at head_dim 64 with one stream: unpadded 128-byte rows
-  // whose 16-byte pieces are permuted by bq_swz (qx below). The S / dP row
-  // reads (16 lanes: 16 consecutive rows, one piece each) and the
-  // transposing reads (32 lanes: 4 consecutive rows x 4 pieces) then meet
-  // 16 distinct 4-bank groups per 16 lanes; with the padded stride the
-  // transposing reads folded rows r and r + 2 onto the same banks. Each
-  // lane's addresses stay loop-invariant.
-  constexpr bool kSwz = D == 64 && !kKV;
-  constexpr int QRS = kSwz ? D : RS;  // row stride of the Q / dO tiles
-  auto qx = [](int row, int e) {      // element offset of (row, feature e)
-    return kSwz ? row * QRS + ((((e >> 3) ^ bq_swz(row)) << 3) | (e & 7)) : row * QRS + e;
+  // Q / dO tiles: unpadded 128-byte rows whose 16-byte pieces are permuted
+  // by bq_swz (qx below). The S / dP row reads (16 lanes: 16 consecutive
+  // rows, one piece each) and the transposing reads (32 lanes: 4 consecutive
+  // rows x 4 pieces) then meet 16 distinct 4-bank groups per 16 lanes; with
+  // padded rows the transposing reads folded rows r and r + 2 onto the same
+  // banks. Each lane's addresses stay loop-invariant.
+  auto qx = [](int row, int e) {  // element offset of (row, feature e)
+    return row * D + ((((e >> 3) ^ bq_swz(row)) << 3) | (e & 7));
   };
   constexpr int KTS = BS + 8;   // row stride of K^T ([d][key])
   // Row stride of dS^T ([key][q]): 34 banks, so the 32 keys of a wave's
   // 8-byte dS writes land on distinct bank pairs (NQ + 8 paired keys c and
   // c + 16; measured 2% faster at 512K).
   constexpr int QS2 = NQ + 4;
-  // K^T ([d][key]) for one stream, or K and V ([key][d]) for two.
-  __shared__ __attribute__((aligned(16))) uint16_t Kl[kKV ? 2 * BS * RS : D * KTS];
-  // Per stream: Q rows, dO rows, dS^T. One array, so that the float32
-  // hand-over of dK / dV between the streams can reuse all of it.
-  constexpr int kRows = 2 * NQ * QRS + BS * QS2;
-  __shared__ __attribute__((aligned(16))) uint16_t Sm[ST * kRows];
-  __shared__ __attribute__((aligned(16))) float s_lse_[ST][NQ];
-  __shared__ __attribute__((aligned(16))) float s_delta_[ST][NQ];
-  __shared__ __attribute__((aligned(16))) int s_lim_[ST][NQ];
+  __shared__ __attribute__((aligned(16))) uint16_t Kt[D * KTS];
+  // Q rows, dO rows, dS^T
+  __shared__ __attribute__((aligned(16))) uint16_t Sm[2 * NQ * D + BS * QS2];
+  __shared__ __attribute__((aligned(16))) float s_lse[NQ];
+  __shared__ __attribute__((aligned(16))) float s_delta[NQ];
+  __shared__ __attribute__((aligned(16))) int s_lim[NQ];
   // dQ destinations by step parity: the stores of step g read them after the
   // dS barrier, while step g + 1's are already being staged.
-  __shared__ int64_t s_dst_[ST][2][NQ];
+  __shared__ int64_t s_dst_[2][NQ];
   // dQ tiles per wave ([q][d], 32 x 32, row stride DQS) on their way out as
   // 16-byte chunks; private to the wave, so only a wave barrier orders them.
   constexpr int TPW = DT * (NQ / 32) / (BS / 32);
   constexpr int DQS = 40;
-  __shared__ __attribute__((aligned(16))) uint16_t DQs_[sizeof(A) == 2 ? ST * (BS / 32) * TPW * 32 * DQS : 8];
-  static_assert((NQ * QRS * 2) % 16 == 0 && (kRows * 2) % 16 == 0, "16-byte aligned carving");
+  __shared__ __attribute__((aligned(16))) uint16_t DQs[sizeof(A) == 2 ? (BS / 32) * TPW * 32 * DQS : 8];
 
   const Column c = resolve_column(a, blockIdx.x, blockIdx.y);
   if (c.skip) return;  // past the segment list (uniform)
@@ -503,18 +522,10 @@ bwd_mfma_kernel(AttnArgs a) {
   if (key_lim <= 0) return;  // uniform
 
   const int lane = tid & 63;
-  const int stream = kKV ? tid / NT : 0;
-  const int stid = kKV ? tid % NT : tid;  // thread index within the stream
-  const int wave = stid >> 6;
-  uint16_t* Qs = Sm + stream * kRows;
-  uint16_t* Os = Qs + NQ * QRS;
-  uint16_t* DSt = Os + NQ * QRS;
-  uint16_t* Kt = Kl;          // one stream
-  uint16_t* Ks = Kl;          // two streams
-  uint16_t* Vs = kKV ? Kl + BS * RS : Kl;  // (unused with one stream)
-  float* s_lse = s_lse_[stream];
-  float* s_delta = s_delta_[stream];
-  int* s_lim = s_lim_[stream];
+  const int wave = tid >> 6;
+  uint16_t* Qs = Sm;
+  uint16_t* Os = Qs + NQ * D;
+  uint16_t* DSt = Os + NQ * D;
   const int h = lane >> 5;
   const int col = lane & 31;
   const int mykey = wave * 32 + col;  // the key this lane holds in S / dP / dV / dK
@@ -523,21 +534,19 @@ bwd_mfma_kernel(AttnArgs a) {
   for (int dt = 0; dt < DT; ++dt) { dv[dt] = floatx16_t{}; dk[dt] = floatx16_t{}; }
   A* dq_out = static_cast<A*>(a.part_acc);
 
-  // Entry pipeline. A thread of the stream's first wave tracks entry
-  // stid % NQ of a step (lanes past NQ duplicate it); its loads are
-  // unconditional within the loop: while step g is computed, the Q / dO
-  // rows and lse / delta of step g + 1 and the index entries of step g + 2
-  // are in flight; everything is waited for once, after the step's dQ.
+  // Entry pipeline. Thread q of the first wave tracks entry q of a step; its
+  // loads are unconditional within the loop: while step g is computed, the
+  // Q / dO rows and lse / delta of step g + 1 and the index entries of step
+  // g + 2 are in flight; everything is waited for once, after the step's dQ.
   constexpr int CH = NQ * D / 8 / NT;  // 16-byte chunks per thread per tensor
   static_assert(NQ * D / 8 % NT == 0, "row chunks must tile the workgroup");
-  const int qi = stid % NQ;
+  const int qi = tid % NQ;
   const int32_t last = c.n > 0 ? c.n - 1 : 0;
   int32_t i_row = 0, i_head = 0, i_slot = 0;    // raw entry, step g + 2
   bool i_live = false;
-  // Only the first wave of a stream (threads stid < 64 >= NQ) loads the
-  // index entries and row statistics, derives them and stages them; the
-  // other waves read what it staged.
-  const bool idx_wave = stid < 64;
+  // Only the first wave loads the index entries and row statistics, derives
+  // them and stages them; the other waves read what it staged.
+  const bool idx_wave = tid < 64;
   auto load_idx = [&](int32_t g) {
     if (!idx_wave) return;  // wave-uniform
     const int32_t e = g + qi;
@@ -551,8 +560,7 @@ bwd_mfma_kernel(AttnArgs a) {
   };
   int64_t n_pr = 0, n_dst = -1;                 // derived, step g + 1
   int n_lim = -1;
-  __shared__ int64_t s_qoff_[ST][NQ];
-  int64_t* s_qoff = s_qoff_[stream];
+  __shared__ int64_t s_qoff[NQ];
   // derive() runs in every wave (on constants outside the first), so the
   // loads above are consumed on every path and never waited for later.
   auto derive = [&]() {
@@ -563,7 +571,7 @@ bwd_mfma_kernel(AttnArgs a) {
     n_pr = ok ? pr : 0;
     n_dst = ok ? pr * a.slots + i_slot : -1;
     n_lim = ok ? min(key_lim - 1, row_lim) : -1;
-    if (stid < NQ) s_qoff[stid] = ok ? q_offset(a, c, i_row, i_head) : -1;
+    if (tid < NQ) s_qoff[tid] = ok ? q_offset(a, c, i_row, i_head) : -1;
   };
   u32x4 pq[CH], po[CH];
   bool pv[CH];  // chunk belongs to a live entry (zeroed when staged)
@@ -576,7 +584,7 @@ bwd_mfma_kernel(AttnArgs a) {
     }
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
-      const int i = stid + u * NT;
+      const int i = tid + u * NT;
       const int64_t o = s_qoff[i / (D / 8)];
       const int64_t off = (o >= 0 ? o : 0) + (i % (D / 8)) * 8;
       pq[u] = *reinterpret_cast<const u32x4*>(Qg + off);
@@ -593,21 +601,20 @@ bwd_mfma_kernel(AttnArgs a) {
   // its entries are in; then K^T is written. Loads are unconditional: keys
   // past the block's end read a valid row (K^T zeroes them; their S and dP
   // are masked and their dK / dV never stored).
-  constexpr int KTN = BS * D / 8 / NTA;  // 16-byte K (and V) chunks per thread
-  static_assert(BS * D / 8 % NTA == 0, "K chunks must tile the workgroup");
-  if (c.n > 0) load_idx(stream * NQ);
-  u32x4 ktc[KTN], vtc[kKV ? KTN : 1];
+  constexpr int KTN = BS * D / 8 / NT;  // 16-byte K (and V) chunks per thread
+  static_assert(BS * D / 8 % NT == 0, "K chunks must tile the workgroup");
+  if (c.n > 0) load_idx(0);
+  u32x4 ktc[KTN];
 #pragma unroll
   for (int u = 0; u < KTN; ++u) {
-    const int i = tid + u * NTA;
+    const int i = tid + u * NT;
     const int key = i / (D / 8);
     const int d8 = (i % (D / 8)) * 8;
     const int64_t off = ((c.tok0 + (key < key_lim ? key : 0)) * a.h_kv + c.hk) * D + d8;
     ktc[u] = *reinterpret_cast<const u32x4*>(Kg + off);
-    if constexpr (kKV) vtc[u] = *reinterpret_cast<const u32x4*>(Vg + off);
   }
-  V8 kb[kKV ? 1 : D / 16], vb[kKV ? 1 : D / 16];
-  if constexpr (!kKV) {
+  V8 kb[D / 16], vb[D / 16];
+  {
     const int64_t off = ((c.tok0 + (mykey < key_lim ? mykey : 0)) * a.h_kv + c.hk) * D + 8 * h;
 #pragma unroll
     for (int k = 0; k < D / 16; ++k) {
@@ -619,22 +626,17 @@ bwd_mfma_kernel(AttnArgs a) {
     derive();
     __syncthreads();
     fetch();
-    load_idx(stream * NQ + ST * NQ);
+    load_idx(NQ);
   }
 #pragma unroll
   for (int u = 0; u < KTN; ++u) {
-    const int i = tid + u * NTA;
+    const int i = tid + u * NT;
     const int key = i / (D / 8);
     const int d8 = (i % (D / 8)) * 8;
     const u32x4 kv = key < key_lim ? ktc[u] : u32x4{0, 0, 0, 0};
-    if constexpr (kKV) {
-      *reinterpret_cast<u32x4*>(&Ks[key * RS + d8]) = kv;
-      *reinterpret_cast<u32x4*>(&Vs[key * RS + d8]) = key < key_lim ? vtc[u] : u32x4{0, 0, 0, 0};
-    } else {
-      const uint16_t* ke = reinterpret_cast<const uint16_t*>(&kv);
+    const uint16_t* ke = reinterpret_cast<const uint16_t*>(&kv);
 #pragma unroll
-      for (int w = 0; w < 8; ++w) Kt[(d8 + w) * KTS + key] = ke[w];
-    }
+    for (int w = 0; w < 8; ++w) Kt[(d8 + w) * KTS + key] = ke[w];
   }
   if (c.n > 0) {
     c_lim = n_lim; c_dst = n_dst; c_lse = n_lse; c_dl = n_dl;
@@ -642,40 +644,36 @@ bwd_mfma_kernel(AttnArgs a) {
   }
   // Stages one step: its limits, row statistics, dQ destinations (parity
   // par) and its Q / dO rows, row-major (the dV / dK products read them
-  // transposed). A dead step (act false) gets zero rows and no entries.
-  auto stage = [&](bool act, int par) {
-    if (stid < NQ) {
-      s_lim[stid] = act ? c_lim : -1;
-      s_lse[stid] = c_lse;
-      s_delta[stid] = c_dl;
-      s_dst_[stream][par][stid] = act ? c_dst : -1;
+  // transposed).
+  auto stage = [&](int par) {
+    if (tid < NQ) {
+      s_lim[tid] = c_lim;
+      s_lse[tid] = c_lse;
+      s_delta[tid] = c_dl;
+      s_dst_[par][tid] = c_dst;
     }
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
-      const int i = stid + u * NT;
+      const int i = tid + u * NT;
       const int q = i / (D / 8);
       const int d8 = (i % (D / 8)) * 8;
-      *reinterpret_cast<u32x4*>(&Qs[qx(q, d8)]) = pv[u] && act ? pq[u] : u32x4{0, 0, 0, 0};
-      *reinterpret_cast<u32x4*>(&Os[qx(q, d8)]) = pv[u] && act ? po[u] : u32x4{0, 0, 0, 0};
+      *reinterpret_cast<u32x4*>(&Qs[qx(q, d8)]) = pv[u] ? pq[u] : u32x4{0, 0, 0, 0};
+      *reinterpret_cast<u32x4*>(&Os[qx(q, d8)]) = pv[u] ? po[u] : u32x4{0, 0, 0, 0};
     }
   };
   // vmcnt(0): the K / V operands and the prologue loads are all resident, so
   // the loop's wait counts start from an empty queue on every path.
   __builtin_amdgcn_s_waitcnt(0x0f70);
-  if (c.n > 0) stage(stream * NQ < c.n, 0);
+  if (c.n > 0) stage(0);
 
-  // Every stream runs the same number of iterations (the barriers are
-  // shared); a stream past the column's end runs a dead step: zero rows,
-  // every entry hidden, nothing stored. Two workgroup barriers per step:
-  // the first makes the step's staging visible (and orders the previous
-  // step's dQ reads of dS^T before this step's dS writes), the second makes
-  // dS visible and frees Qs / Os, which the next step is then staged into
-  // while this step's dQ is formed.
+  // Two workgroup barriers per step: the first makes the step's staging
+  // visible (and orders the previous step's dQ reads of dS^T before this
+  // step's dS writes), the second makes dS visible and frees Qs / Os, which
+  // the next step is then staged into while this step's dQ is formed.
   int par = 0;
-  for (int32_t base = 0; base < c.n; base += ST * NQ, par ^= 1) {
-    const int32_t g0 = base + stream * NQ;
+  for (int32_t base = 0; base < c.n; base += NQ, par ^= 1) {
     __syncthreads();
-    const int64_t* s_dst = s_dst_[stream][par];
+    const int64_t* s_dst = s_dst_[par];
     // Every entry of the step sees the whole block (a strictly past, full
     // block) or is dead: the causal masks can go. A dead entry's Q and dO
     // rows are zero, so it adds nothing to dK / dV either way, and its dQ is
@@ -683,14 +681,13 @@ bwd_mfma_kernel(AttnArgs a) {
     // uniform over the workgroup.
     const bool all_visible = __all(lane >= NQ || s_lim[lane < NQ ? lane : 0] == BS - 1 ||
                                    s_lim[lane < NQ ? lane : 0] < 0);
-    const bool more = g0 + ST * NQ < c.n;
     // Unconditional (past the column's end they read valid, clamped rows
     // and are never used): loads issued under a condition that the
     // consuming derive() below repeats leave the compiler's wait analysis
     // a path on which they are still pending at the next step, and it then
     // waits there for every store in flight.
     fetch();
-    load_idx(g0 + 2 * ST * NQ);
+    load_idx(base + 2 * NQ);
 
     // S and dP for this wave's 32 keys and each 32-query tile; lane <->
     // key, register v <-> query 32 qt + 8(v/4) + 4h + v%4.
@@ -700,13 +697,8 @@ bwd_mfma_kernel(AttnArgs a) {
 #pragma unroll
       for (int k = 0; k < D / 16; ++k) {
         const int qo = qx(qt * 32 + col, 16 * k + 8 * h);
-        if constexpr (kKV) {
-          sacc = M::mma(ld16<V8>(&Qs[qo]), ld16<V8>(&Ks[mykey * RS + 16 * k + 8 * h]), sacc);
-          pacc = M::mma(ld16<V8>(&Os[qo]), ld16<V8>(&Vs[mykey * RS + 16 * k + 8 * h]), pacc);
-        } else {
-          sacc = M::mma(ld16<V8>(&Qs[qo]), kb[k], sacc);
-          pacc = M::mma(ld16<V8>(&Os[qo]), vb[k], pacc);
-        }
+        sacc = M::mma(ld16<V8>(&Qs[qo]), kb[k], sacc);
+        pacc = M::mma(ld16<V8>(&Os[qo]), vb[k], pacc);
       }
       V8 pb[2], db[2];  // P and dS as B operands, K-steps over queries
       auto softmax = [&](auto masked) {
@@ -779,29 +771,17 @@ bwd_mfma_kernel(AttnArgs a) {
       dq[t] = floatx16_t{};
 #pragma unroll
       for (int j = 0; j < BS / 16; ++j) {
-        if constexpr (kKV) {
-          // Both operands by transposing reads with the dV / dK pattern:
-          // lane (col, h) holds, at K slots 8h + 4m + [0, 4), the keys
-          // 16j + 8m + 4h + [0, 4) -- of feature 32dt + col of K (A) and of
-          // query 32qt + col of dS (B).
-          const int kr = 16 * j + 4 * h + ((lane & 15) >> 2);
-          const int c4 = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-          dq[t] = M::mma(ld_tr2<V8>(&Ks[kr * RS + dt * 32 + c4], &Ks[(kr + 8) * RS + dt * 32 + c4]),
-                         ld_tr2<V8>(&DSt[kr * QS2 + qt * 32 + c4], &DSt[(kr + 8) * QS2 + qt * 32 + c4]),
-                         dq[t]);
-        } else {
-          dq[t] = M::mma(ld16<V8>(&Kt[(dt * 32 + col) * KTS + 16 * j + 8 * h]),
-                         ld_tr2<V8>(&DSt[(16 * j + tr_key) * QS2 + qt * 32 + tr_q],
-                                    &DSt[(16 * j + 4 + tr_key) * QS2 + qt * 32 + tr_q]),
-                         dq[t]);
-        }
+        dq[t] = M::mma(ld16<V8>(&Kt[(dt * 32 + col) * KTS + 16 * j + 8 * h]),
+                       ld_tr2<V8>(&DSt[(16 * j + tr_key) * QS2 + qt * 32 + tr_q],
+                                  &DSt[(16 * j + 4 + tr_key) * QS2 + qt * 32 + tr_q]),
+                       dq[t]);
       }
     }
     // dq[t][v] is feature 32dt + 8(v/4) + 4h + v%4 of query 32qt + col.
-    const bool next = base + ST * NQ < c.n;  // uniform: the loop runs again
+    const bool next = base + NQ < c.n;  // uniform: the loop runs again
     if constexpr (sizeof(A) == 2) {
       // dQ through this wave's LDS tiles, read back as 16-byte chunks.
-      uint16_t* dqs = DQs_ + ((stream * NW + wave) * TPW) * 32 * DQS;
+      uint16_t* dqs = DQs + wave * TPW * 32 * DQS;
 #pragma unroll
       for (int t = 0; t < TPW; ++t)
 #pragma unroll
@@ -829,7 +809,7 @@ bwd_mfma_kernel(AttnArgs a) {
       __builtin_amdgcn_sched_barrier(0);
       c_lim = n_lim; c_dst = n_dst; c_lse = n_lse; c_dl = n_dl;
       derive();  // waits for every load in flight
-      if (next) stage(more, par ^ 1);
+      if (next) stage(par ^ 1);
 #pragma unroll
       for (int t = 0; t < TPW; ++t) {
         const int dt = (wave + t * NW) % DT;
@@ -848,7 +828,7 @@ bwd_mfma_kernel(AttnArgs a) {
       __builtin_amdgcn_sched_barrier(0);
       c_lim = n_lim; c_dst = n_dst; c_lse = n_lse; c_dl = n_dl;
       derive();  // waits for every load in flight
-      if (next) stage(more, par ^ 1);
+      if (next) stage(par ^ 1);
 #pragma unroll
       for (int t = 0; t < TPW; ++t) {
         const int tt = wave + t * NW;
@@ -864,93 +844,423 @@ bwd_mfma_kernel(AttnArgs a) {
     }
   }
 
-  if constexpr (kKV) {
-    // Stream 1 hands its float32 sums to stream 0 through the K / V LDS
-    // (free once every step is done), dK then dV; slot (dt, q4, wave, lane)
-    // holds four consecutive floats.
-    float4* xb = reinterpret_cast<float4*>(Kl);
-    static_assert(DT * 4 * NW * 64 * 16 <= sizeof(Kl), "dK / dV hand-over fits the K / V LDS");
-    auto hand_over = [&](floatx16_t (&acc)[DT]) {
-      __syncthreads();  // the previous use of this LDS is complete
-      if (stream == 1) {
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4)
-            xb[((dt * 4 + q4) * NW + wave) * 64 + lane] =
-                make_float4(acc[dt][4 * q4], acc[dt][4 * q4 + 1], acc[dt][4 * q4 + 2], acc[dt][4 * q4 + 3]);
-      }
-      __syncthreads();
-      if (stream == 0) {
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-          for (int q4 = 0; q4 < 4; ++q4) {
-            const float4 o = xb[((dt * 4 + q4) * NW + wave) * 64 + lane];
-            acc[dt][4 * q4] += o.x;
-            acc[dt][4 * q4 + 1] += o.y;
-            acc[dt][4 * q4 + 2] += o.z;
-            acc[dt][4 * q4 + 3] += o.w;
-          }
-      }
-    };
-    hand_over(dk);
-    hand_over(dv);
-    if (stream != 0) return;
-  }
-  // dK, dV of this lane's key: register v is feature 32dt + 8(v/4) + 4h + v%4.
-  // A segment of a cut column leaves its float32 sums in its scratch slot
-  // ([2][BS][D]: dK scaled, dV); the finishing pass adds the column's
-  // segments in order.
-  if (c.nseg > 1) {
-    if (mykey < key_lim) {
-      float* sk = a.seg_scratch +
-                  (static_cast<int64_t>(blockIdx.y) * a.scratch_cap + c.scratch) * 2 * BS * D +
-                  mykey * D + 4 * h;
-      float* sv = sk + BS * D;
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          store4<float>(sk + dt * 32 + 8 * q4, dk[dt][4 * q4] * a.scale,
-                        dk[dt][4 * q4 + 1] * a.scale, dk[dt][4 * q4 + 2] * a.scale,
-                        dk[dt][4 * q4 + 3] * a.scale);
-          store4<float>(sv + dt * 32 + 8 * q4, dv[dt][4 * q4], dv[dt][4 * q4 + 1],
-                        dv[dt][4 * q4 + 2], dv[dt][4 * q4 + 3]);
-        }
+  store_dkv<T, D, BS, DT>(a, c, mykey, key_lim, 4 * h, dk, dv);
+}
+
+// ---------------------------------------------------------------------------
+// Backward at head_dim 128 (bwd_wide_kernel). The products and the semantics
+// are those of bwd_mfma_kernel; the work is split so that a wave holds half a
+// key group's dK / dV. Two waves share each 32 keys: in a step of 64 entries
+// wave `half` forms S, dP, P and dS for query tile `half` (K and V rows of the
+// keys in registers), leaves P and dS in LDS, and after the barrier adds both
+// tiles' contributions to features 64 half .. of dK and dV, its own tile's P
+// and dS from registers and the partner's from LDS.
+//
+// Why: at 128 features the sums of 32 keys take 128 registers. The layout this
+// replaced kept them by reading K and V from LDS: a step of 64 entries moved
+// 512 KiB through a CU's LDS, at least 4096 cycles against 2560 of matrix
+// work, with bank conflicts on the transposing reads on top (blocks under 128
+// keys kept the registers and ran 1 wave per SIMD). This split moves 416 KiB
+// without conflicts: rows of 16 pieces, piece p of row r at p ^ wide_swz(r),
+// where 16 consecutive rows take 16 distinct values (the row reads: 16 rows,
+// one piece each) and rows 4a .. 4a + 3 differ in its upper two bits (the
+// transposing reads: 4 rows x 4 pieces, one 64-byte quarter each). Lane
+// addresses stay loop-invariant up to an XOR with a constant.
+//
+// Bound by the chain of a step (rows -> S, dP -> softmax -> barrier -> dV, dK,
+// dQ) at 2 waves per SIMD. [1, 32768, 32 query / 8 kv, 128], 128-key blocks,
+// top_k 8: 2392 -> 2035 us (630 TFLOP/s of its five products); [8, 4096, 16 /
+// 4, 128], 64 keys, top_k 4: 612 -> 498; [2, 8192, 8, 128], 32 keys: 282 ->
+// 235. A register spilled in the loop costs more than anything else here: its
+// reload waits for the rows in flight (24 of them: 3290 us).
+// ---------------------------------------------------------------------------
+__device__ constexpr int wide_swz(int row) { return ((row & 3) << 2) | ((row >> 2) & 3); }
+
+template <typename T, typename A, int BS>
+__global__ void __launch_bounds__(4 * BS, BS == 32 ? 1 : 2)
+bwd_wide_kernel(AttnArgs a) {
+  using M = Mfma<T>;
+  using V8 = typename M::vec;
+  using Sc = typename M::scalar;
+  constexpr int D = 128;
+  constexpr int NQ = 64;
+  constexpr int NW = BS / 16;   // waves: two per 32 keys
+  constexpr int NT = 64 * NW;
+  constexpr int KTS = BS + 8;   // row stride of K^T ([d][key])
+  constexpr int QS = NQ + 4;    // row stride of P^T and dS^T ([key][q]), as QS2 of bwd_mfma_kernel
+  constexpr int TPW = 8 / NW;   // dQ tiles (32 features x 32 queries) per wave
+  constexpr int DQS = 40;
+  __shared__ __attribute__((aligned(16))) uint16_t Kt[D * KTS];
+  // Q and dO rows, then P^T and dS^T: each pair one array, so that one lane
+  // address serves both.
+  // With 128 keys, where one workgroup fills the CU either way, two buffers
+  // of rows by step parity, so that staging the next step waits for no wave.
+  constexpr int QB = BS == 128 ? 2 : 1;
+  // At 64 keys the rows in flight (32 registers per lane) leave no room for
+  // values that could be made again or fetched later.
+  constexpr bool kTight = BS == 64;
+  __shared__ __attribute__((aligned(16))) uint16_t Qs[QB * 2 * NQ * D];
+  __shared__ __attribute__((aligned(16))) uint16_t Pt[2 * BS * QS];
+  uint16_t* const DSt = Pt + BS * QS;
+  // One dQ tile per wave ([q][d]) on its way out as 16-byte chunks.
+  __shared__ __attribute__((aligned(16))) uint16_t DQ[sizeof(A) == 2 ? NW * 32 * DQS : 8];
+  __shared__ __attribute__((aligned(16))) float s_lse[NQ], s_delta[NQ];
+  __shared__ __attribute__((aligned(16))) int s_lim[NQ];
+  __shared__ int64_t s_dst_[2][NQ];  // dQ destinations by step parity
+  __shared__ int64_t s_qoff[NQ];
+
+  const Column c = resolve_column(a, blockIdx.x, blockIdx.y);
+  if (c.skip) return;  // past the segment list (uniform)
+  const int key_lim = static_cast<int>(c.key_end - c.key0);
+  if (key_lim <= 0) return;  // a column past its sequence: its rows lie past the tensor (uniform)
+  const uint16_t* Kg = static_cast<const uint16_t*>(a.k);
+  const uint16_t* Vg = static_cast<const uint16_t*>(a.v);
+  const uint16_t* Qg = static_cast<const uint16_t*>(a.q);
+  const uint16_t* Og = static_cast<const uint16_t*>(a.dout);
+  A* dq_out = static_cast<A*>(a.part_acc);
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = tid >> 6;
+  const int half = wave & 1;
+  const int h = lane >> 5;
+  const int col = lane & 31;
+  const int mykey = (wave >> 1) * 32 + col;  // the key this lane holds in S / dP / dV / dK
+
+  // Entry pipeline, as in bwd_mfma_kernel: the first wave tracks the step's
+  // entries; while step g is computed, the rows and row statistics of step
+  // g + 1 and the index entries of step g + 2 are in flight.
+  constexpr int CH = NQ * D / 8 / NT;  // 16-byte chunks per thread per tensor
+  const int qi = tid % NQ;
+  const int32_t last = c.n > 0 ? c.n - 1 : 0;
+  int32_t i_row = 0, i_head = 0, i_slot = 0;
+  bool i_live = false;
+  const bool idx_wave = tid < 64;
+  auto load_idx = [&](int32_t g) {
+    if (!idx_wave) return;  // wave-uniform
+    const int32_t e = g + qi;
+    const int64_t i = c.lo + (e < c.n ? e : last);
+    i_row = a.row_indices[i * a.istride];
+    i_head = a.head_indices[i * a.istride];
+    i_slot = a.slot_of_pair[i * a.istride];
+    i_live = e < c.n;
+  };
+  int64_t n_pr = 0, n_dst = -1;
+  int n_lim = -1;
+  // Runs in every wave (on constants outside the first), so the index loads
+  // are consumed on every path and never waited for later.
+  auto derive = [&]() {
+    const bool ok = i_live;
+    const int64_t pr = part_row(a, c, i_row, i_head);
+    const int64_t rrel = static_cast<int64_t>(i_row) - c.key0;
+    const int row_lim = !a.causal ? BS : (rrel < 0 ? -1 : (rrel >= BS ? BS : static_cast<int>(rrel)));
+    n_pr = ok ? pr : 0;
+    n_dst = ok ? pr * a.slots + i_slot : -1;
+    n_lim = ok ? min(key_lim - 1, row_lim) : -1;
+    if (idx_wave) s_qoff[tid] = ok ? q_offset(a, c, i_row, i_head) : -1;
+  };
+  u32x4 pq[CH], po[CH];
+  bool pv[CH];  // chunk belongs to a live entry (zeroed when staged)
+  float n_lse = 0.f, n_dl = 0.f;
+  auto fetch_stats = [&]() {
+    if (idx_wave) {
+      const float2 ld = *reinterpret_cast<const float2*>(a.lse_delta + 2 * n_pr);
+      n_lse = ld.x;
+      n_dl = ld.y;
     }
-    return;
+  };
+  auto fetch_rows = [&](int u0, int u1) {
+#pragma unroll
+    for (int u = u0; u < u1; ++u) {
+      const int i = tid + u * NT;
+      const int64_t o = s_qoff[i / (D / 8)];
+      const int64_t off = (o >= 0 ? o : 0) + (i % (D / 8)) * 8;
+      pq[u] = *reinterpret_cast<const u32x4*>(Qg + off);
+      po[u] = *reinterpret_cast<const u32x4*>(Og + off);
+      pv[u] = o >= 0;
+    }
+  };
+  int c_lim = -1;
+  int64_t c_dst = -1;
+  float c_lse = 0.f, c_dl = 0.f;
+  auto stage = [&](int par) {
+    if (idx_wave) {
+      s_lim[tid] = c_lim;
+      s_lse[tid] = c_lse;
+      s_delta[tid] = c_dl;
+      s_dst_[par][tid] = c_dst;
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int i = tid + u * NT;
+      const int q = i / (D / 8);
+      uint16_t* p = Qs + (QB - 1) * par * 2 * NQ * D + q * D + (((i % (D / 8)) ^ wide_swz(q)) << 3);
+      *reinterpret_cast<u32x4*>(p) = pv[u] ? pq[u] : u32x4{0, 0, 0, 0};
+      *reinterpret_cast<u32x4*>(p + NQ * D) = pv[u] ? po[u] : u32x4{0, 0, 0, 0};
+    }
+  };
+
+  // Column start: K^T to LDS (keys past the end zero), this lane's key's K
+  // and V rows to registers (past the end a valid row: its S and dP are
+  // masked and its dK / dV never stored).
+  constexpr int KTN = BS * D / 8 / NT;
+  if (c.n > 0) load_idx(0);
+  u32x4 ktc[KTN];
+#pragma unroll
+  for (int u = 0; u < KTN; ++u) {
+    const int i = tid + u * NT;
+    const int key = i / (D / 8);
+    ktc[u] = *reinterpret_cast<const u32x4*>(
+        Kg + ((c.tok0 + (key < key_lim ? key : 0)) * a.h_kv + c.hk) * D + (i % (D / 8)) * 8);
   }
-  if (mykey < key_lim) {
-    const int64_t off = ((c.tok0 + mykey) * a.h_kv + c.hk) * D + 4 * h;
-    auto store_kv = [&](auto* dK, auto* dV) {
-      using E = std::remove_pointer_t<decltype(dK)>;
+  V8 kb[D / 16], vb[D / 16];
+  {
+    const int64_t off = ((c.tok0 + (mykey < key_lim ? mykey : 0)) * a.h_kv + c.hk) * D + 8 * h;
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
+    for (int k = 0; k < D / 16; ++k) {
+      kb[k] = ld16<V8>(Kg + off + 16 * k);
+      vb[k] = ld16<V8>(Vg + off + 16 * k);
+    }
+  }
+  floatx16_t dv[2], dk[2];
 #pragma unroll
-        for (int q4 = 0; q4 < 4; ++q4) {
-          store4<E>(dK + dt * 32 + 8 * q4, dk[dt][4 * q4] * a.scale, dk[dt][4 * q4 + 1] * a.scale,
-                    dk[dt][4 * q4 + 2] * a.scale, dk[dt][4 * q4 + 3] * a.scale);
-          store4<E>(dV + dt * 32 + 8 * q4, dv[dt][4 * q4], dv[dt][4 * q4 + 1],
-                    dv[dt][4 * q4 + 2], dv[dt][4 * q4 + 3]);
+  for (int dt = 0; dt < 2; ++dt) { dv[dt] = floatx16_t{}; dk[dt] = floatx16_t{}; }
+  if (c.n > 0) {
+    derive();
+    __syncthreads();
+    fetch_stats();
+    fetch_rows(0, CH);
+    load_idx(NQ);
+  }
+#pragma unroll
+  for (int u = 0; u < KTN; ++u) {
+    const int i = tid + u * NT;
+    const int key = i / (D / 8);
+    const int d8 = (i % (D / 8)) * 8;
+    const u32x4 kv = key < key_lim ? ktc[u] : u32x4{0, 0, 0, 0};
+    const uint16_t* ke = reinterpret_cast<const uint16_t*>(&kv);
+#pragma unroll
+    for (int w = 0; w < 8; ++w) Kt[(d8 + w) * KTS + key] = ke[w];
+  }
+  if (c.n > 0) {
+    c_lim = n_lim; c_dst = n_dst; c_lse = n_lse; c_dl = n_dl;
+    __syncthreads();  // every thread has read step 0's s_qoff
+    derive();
+  }
+  // vmcnt(0): the loop's wait counts start from an empty queue on every path.
+  __builtin_amdgcn_s_waitcnt(0x0f70);
+  if (c.n > 0) stage(0);
+
+  // Two barriers per step: the first makes the step's staging visible (and
+  // orders the previous step's reads of P and dS before this step's writes),
+  // the second makes P and dS visible.
+  int par = 0;
+  for (int32_t base = 0; base < c.n; base += NQ, par ^= 1) {
+    __syncthreads();
+    const int64_t* s_dst = s_dst_[par];
+    // Every entry sees the whole block or is dead: no causal masks.
+    const int lim = s_lim[lane];
+    const bool all_visible = __all(lim == BS - 1 || lim < 0);
+    // Unconditional (past the column's end clamped, valid rows). With four or
+    // more chunks per thread half of them wait until S and dP have left their
+    // registers.
+    constexpr int C0 = kTight ? CH / 2 : CH;
+    fetch_stats();
+    fetch_rows(0, C0);
+    load_idx(base + 2 * NQ);
+
+    // What is opaque in every step is made again where it is used: the
+    // XORed addresses from their lane's base (one instruction each), at 64
+    // keys every LDS address from the lane number. Hoisted out of the loop
+    // they would push operands out of the registers.
+    int ln = lane;
+    if constexpr (kTight) asm volatile("" : "+v"(ln));
+    // Row reads: piece 2k + h of row col of the own tile (elements).
+    int r_row = (32 * half + (ln & 31)) * D + (((ln >> 5) ^ wide_swz(ln & 31)) << 3);
+    asm volatile("" : "+v"(r_row));
+    const uint16_t* rows = Qs + (QB - 1) * par * 2 * NQ * D;
+    floatx16_t sacc = floatx16_t{}, pacc = floatx16_t{};
+    {
+#pragma unroll
+      for (int k = 0; k < D / 16; ++k) {
+        const uint16_t* p = rows + (r_row ^ (k << 4));
+        sacc = M::mma(ld16<V8>(p), kb[k], sacc);
+        pacc = M::mma(ld16<V8>(p + NQ * D), vb[k], pacc);
+      }
+    }
+    V8 pb[2], db[2];  // own tile's P and dS as B operands, K-steps over queries
+    auto softmax = [&](auto masked) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {  // queries 32 half + 8g + 4h + [0, 4)
+        const int q0 = 32 * half + 8 * g + 4 * h;
+        int limv[4] = {BS, BS, BS, BS};
+        if constexpr (decltype(masked)::value) {
+          const int4 lim4 = *reinterpret_cast<const int4*>(&s_lim[q0]);
+          limv[0] = lim4.x; limv[1] = lim4.y; limv[2] = lim4.z; limv[3] = lim4.w;
         }
+        const float4 lse4 = *reinterpret_cast<const float4*>(&s_lse[q0]);
+        const float4 dl4 = *reinterpret_cast<const float4*>(&s_delta[q0]);
+        const float lsev[4] = {lse4.x, lse4.y, lse4.z, lse4.w};
+        const float dlv[4] = {dl4.x, dl4.y, dl4.z, dl4.w};
+        typedef Sc sc4_t __attribute__((ext_vector_type(4)));
+        typedef float f32x4_t __attribute__((ext_vector_type(4)));
+        f32x4_t pf, dsf;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          const int v = 4 * g + w;
+          const float x = (!decltype(masked)::value || mykey <= limv[w])
+                              ? sacc[v] * a.scale_log2 - lsev[w] : -INFINITY;
+          pf[w] = __builtin_amdgcn_exp2f(x);
+          dsf[w] = pf[w] * (pacc[v] - dlv[w]);
+        }
+        const sc4_t p4 = __builtin_convertvector(pf, sc4_t);
+        const sc4_t d4 = __builtin_convertvector(dsf, sc4_t);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+          pb[g >> 1][4 * (g & 1) + w] = p4[w];
+          db[g >> 1][4 * (g & 1) + w] = d4[w];
+        }
+        *reinterpret_cast<uint2*>(&Pt[mykey * QS + q0]) = __builtin_bit_cast(uint2, p4);
+        *reinterpret_cast<uint2*>(&DSt[mykey * QS + q0]) = __builtin_bit_cast(uint2, d4);
+      }
     };
-    if (a.dkv_f32)  // uniform: float32 sums for a caller that adds several calls
-      store_kv(static_cast<float*>(a.dk) + off, static_cast<float*>(a.dv) + off);
-    else
-      store_kv(static_cast<T*>(a.dk) + off, static_cast<T*>(a.dv) + off);
+    if (all_visible) softmax(std::false_type{});
+    else softmax(std::true_type{});
+    __syncthreads();  // P and dS of every wave visible
+    fetch_rows(C0, CH);
+
+    // dV^T += dO^T . P and dK^T += Q^T . dS on this wave's features, the own
+    // tile first (A operands as in bwd_mfma_kernel). Transposing reads of half
+    // m of an operand: row tr_row + 8m, pieces of those features.
+    if constexpr (kTight) asm volatile("" : "+v"(ln));
+    const int tr_row = 4 * (ln >> 5) + ((ln & 15) >> 2);
+    const int tr_piece = 8 * half + 2 * ((ln >> 4) & 1) + ((ln & 3) >> 1);
+    int r_tr0 = tr_row * D + ((tr_piece ^ wide_swz(tr_row)) << 3) + 4 * (ln & 1);
+    int r_tr1 = (tr_row + 8) * D + ((tr_piece ^ wide_swz(tr_row + 8)) << 3) + 4 * (ln & 1);
+    asm volatile("" : "+v"(r_tr0), "+v"(r_tr1));
+    auto add_tile = [&](int qt, const V8 (&p)[2], const V8 (&d)[2]) {
+      const uint16_t* tile = rows + 32 * qt * D;
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int dt = 0; dt < 2; ++dt) {
+          const uint16_t* p0 = tile + (r_tr0 ^ (dt << 5)) + 16 * j * D;
+          const uint16_t* p1 = tile + (r_tr1 ^ (dt << 5)) + 16 * j * D;
+          dv[dt] = M::mma(ld_tr2<V8>(p0 + NQ * D, p1 + NQ * D), p[j], dv[dt]);
+          dk[dt] = M::mma(ld_tr2<V8>(p0, p1), d[j], dk[dt]);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    add_tile(half, pb, db);
+    {
+      // The partner's: queries 16j + 8m + 4h + [0, 4) of its tile are K slots
+      // 4m + [0, 4).
+      const int q0 = ((wave >> 1) * 32 + (ln & 31)) * QS + 32 * (half ^ 1) + 4 * (ln >> 5);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const uint2 p0 = *reinterpret_cast<const uint2*>(&Pt[q0 + 16 * j]);
+        const uint2 p1 = *reinterpret_cast<const uint2*>(&Pt[q0 + 16 * j + 8]);
+        const uint2 d0 = *reinterpret_cast<const uint2*>(&DSt[q0 + 16 * j]);
+        const uint2 d1 = *reinterpret_cast<const uint2*>(&DSt[q0 + 16 * j + 8]);
+        pb[j] = __builtin_bit_cast(V8, u32x4{p0.x, p0.y, p1.x, p1.y});
+        db[j] = __builtin_bit_cast(V8, u32x4{d0.x, d0.y, d1.x, d1.y});
+      }
+    }
+    add_tile(half ^ 1, pb, db);
+
+    // dQ^T[d][q] over all keys, tiles spread over the waves; operands as in
+    // bwd_mfma_kernel.
+    if constexpr (kTight) asm volatile("" : "+v"(ln));
+    const int tr_key = 8 * (ln >> 5) + ((ln & 15) >> 2);
+    const int tr_q = 16 * ((ln >> 4) & 1) + 4 * (ln & 3);
+    floatx16_t dq[TPW];
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+      const int tt = wave + t * NW;
+      const int dt = tt & 3, qt = tt >> 2;
+      dq[t] = floatx16_t{};
+#pragma unroll
+      for (int j = 0; j < BS / 16; ++j)
+        dq[t] = M::mma(ld16<V8>(&Kt[(dt * 32 + (ln & 31)) * KTS + 16 * j + 8 * (ln >> 5)]),
+                       ld_tr2<V8>(&DSt[(16 * j + tr_key) * QS + qt * 32 + tr_q],
+                                  &DSt[(16 * j + 4 + tr_key) * QS + qt * 32 + tr_q]),
+                       dq[t]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // dq[t][v] is feature 32dt + 8(v/4) + 4h + v%4 of query 32qt + col.
+    const bool next = base + NQ < c.n;  // uniform
+    u32x4 val[TPW][2];
+    int64_t dst[TPW][2];
+    auto load_dst = [&](int t) {
+      const int64_t* d = s_dst + ((wave + t * NW) >> 2) * 32;
+      dst[t][0] = d[sizeof(A) == 2 ? ln >> 2 : ln & 31];
+      dst[t][1] = d[16 + (ln >> 2)];
+    };
+    if constexpr (!kTight)
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) load_dst(t);
+    if constexpr (sizeof(A) == 2) {
+      uint16_t* dqs = DQ + wave * 32 * DQS;
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) {
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4)
+          store4<A>(reinterpret_cast<A*>(&dqs[(ln & 31) * DQS + 8 * q4 + 4 * (ln >> 5)]),
+                    dq[t][4 * q4] * a.scale, dq[t][4 * q4 + 1] * a.scale,
+                    dq[t][4 * q4 + 2] * a.scale, dq[t][4 * q4 + 3] * a.scale);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int ci = ln + 64 * u;
+          val[t][u] = *reinterpret_cast<const u32x4*>(&dqs[(ci >> 2) * DQS + (ci & 3) * 8]);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      }
+    }
+    // Keep the next step's index arithmetic (which waits for the loads in
+    // flight) behind this step's work.
+    __builtin_amdgcn_sched_barrier(0);
+    c_lim = n_lim; c_dst = n_dst; c_lse = n_lse; c_dl = n_dl;
+    if (QB == 1 && next) __syncthreads();  // the rows are read
+    if constexpr (kTight) {
+      if (next) stage(par ^ 1);
+      derive();
+    } else {
+      derive();  // waits for every load in flight
+      if (next) stage(par ^ 1);
+    }
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) {
+      const int dt = (wave + t * NW) & 3;
+      if constexpr (kTight) load_dst(t);
+      if constexpr (sizeof(A) == 2) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+          if (dst[t][u] >= 0)
+            *reinterpret_cast<u32x4*>(dq_out + dst[t][u] * D + dt * 32 + (lane & 3) * 8) = val[t][u];
+      } else if (dst[t][0] >= 0) {
+        A* p = dq_out + dst[t][0] * D + dt * 32 + 4 * h;
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4)
+          store4<A>(p + 8 * q4, dq[t][4 * q4] * a.scale, dq[t][4 * q4 + 1] * a.scale,
+                    dq[t][4 * q4 + 2] * a.scale, dq[t][4 * q4 + 3] * a.scale);
+      }
+    }
   }
+
+  store_dkv<T, D, BS, 2>(a, c, mykey, key_lim, 64 * half + 4 * h, dk, dv);
 }
 
 template <typename T, typename A, int D, int BS>
 static int launch_bwd(const AttnArgs& a, int64_t n_cols, hipStream_t st) {
-  // 64 queries per step at head_dim 64, 32 at 128 (wider steps spill). At
-  // head_dim 128 with 128-key blocks, two streams of 4 waves share the keys
-  // (K / V in LDS): 8 waves, 2 per SIMD, in 125 KiB of LDS.
-  constexpr int ST = (D == 128 && BS == 128) ? 2 : 1;
-  constexpr int NQ = D == 128 ? 32 : 64;
   dim3 grid(static_cast<unsigned>(a.seg ? a.seg_cap : a.n_blocks), static_cast<unsigned>(n_cols));
-  hipLaunchKernelGGL((bwd_mfma_kernel<T, A, D, BS, NQ, ST>), grid, dim3(BS * 2 * ST), 0, st, a);
+  if constexpr (D == 128)
+    hipLaunchKernelGGL((bwd_wide_kernel<T, A, BS>), grid, dim3(4 * BS), 0, st, a);
+  else
+    hipLaunchKernelGGL((bwd_mfma_kernel<T, A, BS>), grid, dim3(BS * 2), 0, st, a);
   return check_launch("moba_bwd (mfma)");
 }
 
