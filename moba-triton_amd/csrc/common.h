@@ -127,11 +127,15 @@ int make_geometry(Geometry* g, int64_t batch, int64_t seq_len,
                   int64_t head_dim, int64_t n_blocks, int64_t block_size,
                   int64_t slots, const int32_t* cu_seqlens);
 
-// The gate on float64 matrix products (gate_f64.hip): whether it takes the
-// call, and the call.
-bool gate_f64_takes(const void* q, const void* kbar, const Geometry& g, int take, int dtype);
+// Queries per tile of the approximate gate kernel.
+constexpr int kGateTile = 128;
+
+// The gate on float64 matrix products (gate_f64.hip): how many positions from
+// the start of every sequence it takes (all rows_per_seq of them, none, or a
+// multiple of kGateTile), and the call over `rows` of them.
+int64_t gate_f64_rows(const void* q, const void* kbar, const Geometry& g, int take, int dtype);
 int gate_f64(const void* q, const void* kbar, int32_t* out, const int32_t* cu, const Geometry& g,
-             int take, int cur, int dtype, hipStream_t st);
+             int64_t rows, int take, int cur, int dtype, hipStream_t st);
 
 // Device view of where a sequence lives. Padded: sequence r is batch row r,
 // tokens [r*S, r*S + S). Packed: tokens [cu[r], cu[r+1]).

@@ -67,8 +67,8 @@
 //   thread per query, exact float64 scores for every candidate, streaming
 //   top-T in registers.
 //
-// Calls with few blocks per row, and float32 at head_dim 64 / 128, run
-// gate_f64.hip instead.
+// Calls with few blocks per row, the first positions of calls with long lists
+// and more blocks, and float32 at head_dim 64 / 128, run gate_f64.hip instead.
 #include "common.h"
 
 #include <mutex>
@@ -1678,7 +1678,7 @@ static int dispatch_exact(const void* q, const void* kbar, int32_t* out,
 
 template <typename T, int D, int M>
 static int launch_mfma(const void* q, const void* kbar, int32_t* out, const int32_t* cu,
-                       const Geometry& g, int take, int cur, const GateWs& ws,
+                       const Geometry& g, int64_t first, int take, int cur, const GateWs& ws,
                        hipStream_t st) {
   // Groups of 4 blocks, 4 waves (3 workgroups per CU at head_dim 64).
   // Groups of 8 at 8 waves per workgroup (2 per SIMD, the records need
@@ -1692,7 +1692,10 @@ static int launch_mfma(const void* q, const void* kbar, int32_t* out, const int3
   // finds its candidates outside the kept groups about once in 4e4.
   constexpr int K = M <= 12 ? 8 : 16;
   const FbLists fb{ws.fb_list, ws.fb_count, ws.fb_cap};
-  dim3 grid(static_cast<unsigned>(cdiv(g.rows_per_seq, 32 * WAVES)),
+  // Positions from `first`, a multiple of the tile: the kernel numbers its
+  // tiles from the end.
+  static_assert(32 * WAVES == kGateTile, "the split falls between tiles");
+  dim3 grid(static_cast<unsigned>(cdiv(g.rows_per_seq, 32 * WAVES) - first / (32 * WAVES)),
             static_cast<unsigned>(g.rows * g.h_q));
   hipLaunchKernelGGL((gate_mfma_kernel<T, D, M, K, CAP, WAVES, GB>), grid, dim3(64 * WAVES), 0, st,
                      static_cast<const T*>(q), static_cast<const T*>(kbar), out, cu,
@@ -1732,8 +1735,8 @@ static int run_gate(const void* q, const void* kbar, int32_t* out, const int32_t
                     size_t ws_bytes, hipStream_t st) {
   if constexpr (Elem<T>::kCode == MOBA_FP32) {
     (void)workspace; (void)ws_bytes;
-    if (gate_f64_takes(q, kbar, g, take, MOBA_FP32))
-      return gate_f64(q, kbar, out, cu, g, take, cur, MOBA_FP32, st);
+    if (gate_f64_rows(q, kbar, g, take, MOBA_FP32) == g.rows_per_seq)
+      return gate_f64(q, kbar, out, cu, g, g.rows_per_seq, take, cur, MOBA_FP32, st);
     return dispatch_exact<T>(q, kbar, out, cu, g, take, cur, nullptr, nullptr, st);
   } else {
   // Block ids travel through LDS as 16 bits in the MFMA kernel.
@@ -1744,8 +1747,13 @@ static int run_gate(const void* q, const void* kbar, int32_t* out, const int32_t
   if (!workspace || ws_bytes < moba_gate_workspace_size(g.rows, g.rows_per_seq, g.h_q) ||
       ws_bytes < ws.bytes)
     return fail(MOBA_ERR_WORKSPACE, "gate workspace too small");
-  if (gate_f64_takes(q, kbar, g, take, Elem<T>::kCode))
-    return gate_f64(q, kbar, out, cu, g, take, cur, Elem<T>::kCode, st);
+  // The first f64_rows positions of every sequence by exact products, the
+  // rest by the kernels below.
+  const int64_t f64_rows = gate_f64_rows(q, kbar, g, take, Elem<T>::kCode);
+  if (f64_rows > 0) {
+    int rc = gate_f64(q, kbar, out, cu, g, f64_rows, take, cur, Elem<T>::kCode, st);
+    if (rc || f64_rows == g.rows_per_seq) return rc;
+  }
   unsigned* norm_bits = reinterpret_cast<unsigned*>(ws.kbar_norm);
   hipLaunchKernelGGL(gate_init_kernel, dim3(1), dim3(256), 0, st, norm_bits,
                      g.rows * g.h_kv, ws.counter, ws.fb_count, g.rows * g.h_q * kFbBuckets);
@@ -1757,11 +1765,11 @@ static int run_gate(const void* q, const void* kbar, int32_t* out, const int32_t
   int rc = check_launch("moba_gate (prep)");
   if (rc) return rc;
   if (g.head_dim == 64) {
-    rc = take <= 8 ? launch_mfma<T, 64, 12>(q, kbar, out, cu, g, take, cur, ws, st)
-                   : launch_mfma<T, 64, 20>(q, kbar, out, cu, g, take, cur, ws, st);
+    rc = take <= 8 ? launch_mfma<T, 64, 12>(q, kbar, out, cu, g, f64_rows, take, cur, ws, st)
+                   : launch_mfma<T, 64, 20>(q, kbar, out, cu, g, f64_rows, take, cur, ws, st);
   } else {
-    rc = take <= 8 ? launch_mfma<T, 128, 12>(q, kbar, out, cu, g, take, cur, ws, st)
-                   : launch_mfma<T, 128, 20>(q, kbar, out, cu, g, take, cur, ws, st);
+    rc = take <= 8 ? launch_mfma<T, 128, 12>(q, kbar, out, cu, g, f64_rows, take, cur, ws, st)
+                   : launch_mfma<T, 128, 20>(q, kbar, out, cu, g, f64_rows, take, cur, ws, st);
   }
   if (rc) return rc;
   // Queries whose approximate evidence was insufficient: exact rescoring,

@@ -27,7 +27,7 @@
 // score and SIMD at head_dim 64 / 128), several times the cost per score of
 // the approximate kernel of gate.hip, against that kernel's cost per query
 // (lists, classification and rescoring of candidates, six launches).
-// gate_f64_takes() below draws the line.
+// gate_f64_rows() below draws the line.
 #include "common.h"
 
 namespace moba {
@@ -261,8 +261,8 @@ gate_f64_kernel(const T* __restrict__ q, const T* __restrict__ kbar, int32_t* __
 
 template <typename T, int D>
 int launch(const void* q, const void* kbar, int32_t* out, const int32_t* cu, const Geometry& g,
-           int take, int cur, hipStream_t st) {
-  const dim3 grid(static_cast<unsigned>(cdiv(g.rows_per_seq, 16 * kWaves)),
+           int64_t rows, int take, int cur, hipStream_t st) {
+  const dim3 grid(static_cast<unsigned>(cdiv(rows, 16 * kWaves)),
                   static_cast<unsigned>(g.rows * g.h_q));
   auto go = [&](auto kern) {
     hipLaunchKernelGGL(kern, grid, dim3(64 * kWaves), 0, st, static_cast<const T*>(q),
@@ -289,20 +289,33 @@ int launch(const void* q, const void* kbar, int32_t* out, const int32_t* cu, con
 // by one); head_dim 128: 135 against 147 / 179, 164 / 233, 419 / 523.
 // float32 has no approximate kernel: 64K queries of 127 blocks take 33 us
 // (head_dim 64) and 54 us (128), and took 1330 and 2400 in gate_exact_kernel.
-bool gate_f64_takes(const void* q, const void* kbar, const Geometry& g, int take, int dtype) {
-  if ((g.head_dim != 64 && g.head_dim != 128) || take > 16 || g.rows * g.h_q > 65535) return false;
+//
+// With lists of 9 to 16 and more blocks than that, the line is drawn per
+// position instead of per call: the cost here grows with a query's past
+// blocks, the approximate kernels' hardly does. Measured over lists of 9 to 16
+// and both 16-bit types: 128K queries of 256 blocks 128 .. 294 us whole and
+// 116 .. 226 split (head_dim 64 and 128), 156K of 313 blocks 146 .. 347 and
+// 139 .. 287, 512K of 512 blocks 450 .. 1167 and 380 .. 1019. The two parts
+// run one after the other, so a split pays only where the first part fills
+// the chip by itself: 61K queries of it (512K of 2048 blocks) are even, 41K
+// (125K of 400, head_dim 128) lose 1% on some keys, 7K (8K of 256) 15 us.
+int64_t gate_f64_rows(const void* q, const void* kbar, const Geometry& g, int take, int dtype) {
+  if ((g.head_dim != 64 && g.head_dim != 128) || take > 16 || g.rows * g.h_q > 65535) return 0;
   // Rows are read in 16-byte pieces.
-  if ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(kbar)) & 15) return false;
-  if (dtype == MOBA_FP32) return true;
-  if (take > 8) return g.n_blocks < 256;
-  return g.n_blocks <= (g.head_dim == 64 ? 96 : 64);
+  if ((reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(kbar)) & 15) return 0;
+  if (dtype == MOBA_FP32) return g.rows_per_seq;
+  if (take <= 8) return g.n_blocks <= (g.head_dim == 64 ? 96 : 64) ? g.rows_per_seq : 0;
+  if (g.n_blocks < 256) return g.rows_per_seq;
+  const int64_t rows = (g.head_dim == 64 ? 240 : 128) * g.block_size / kGateTile * kGateTile;
+  const int64_t part = rows < g.rows_per_seq ? rows : g.rows_per_seq;
+  return g.rows * g.h_q * part >= 65536 ? part : 0;
 }
 
 int gate_f64(const void* q, const void* kbar, int32_t* out, const int32_t* cu, const Geometry& g,
-             int take, int cur, int dtype, hipStream_t st) {
+             int64_t rows, int take, int cur, int dtype, hipStream_t st) {
   return MOBA_DISPATCH_DTYPE(dtype, T, [&] {
-    return g.head_dim == 64 ? launch<T, 64>(q, kbar, out, cu, g, take, cur, st)
-                            : launch<T, 128>(q, kbar, out, cu, g, take, cur, st);
+    return g.head_dim == 64 ? launch<T, 64>(q, kbar, out, cu, g, rows, take, cur, st)
+                            : launch<T, 128>(q, kbar, out, cu, g, rows, take, cur, st);
   });
 }
 

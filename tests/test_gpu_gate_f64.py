@@ -37,6 +37,13 @@ def _padded(kbar, n):
     return torch.cat((kbar, pad), 2).contiguous()
 
 
+def _shifted(t):
+    """The same values off a 16-byte boundary: the approximate kernels."""
+    buf = torch.empty(t.numel() + 4, device=t.device, dtype=t.dtype)
+    buf[4:] = t.reshape(-1)
+    return buf[4:].view(t.shape)
+
+
 # (S, query heads, kv heads, head_dim, block, top_k): one query, one block,
 # a tile of 16 blocks or queries less / exactly / plus one, the last block
 # counts of the rule, list lengths 1, 4, 5, 8, 9 and 16 and slots left over.
@@ -61,6 +68,7 @@ def test_gate_f64_matches_oracle_and_general_path(device, case, dtype):
     assert torch.equal(got.cpu(), ref)
     if dtype != torch.float32:
         assert torch.equal(got, _gate(q, _padded(kbar, 300), cfg, s, take))
+        assert torch.equal(got, _gate(_shifted(q), kbar, cfg, s, take))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -88,3 +96,35 @@ def test_gate_f64_special_values_match_general_path(device, kind, dtype):
     take = cfg.past_blocks_selected(44)
     got = _gate(q, kbar, cfg, max(lens), take, cu)
     assert torch.equal(got, _gate(q, _padded(kbar, 300), cfg, max(lens), take, cu))
+
+
+# With lists over 8 and 256 blocks or more, the first 240 (head_dim 64) or 128
+# blocks' queries, to a whole 128-query tile, go to these kernels and the rest
+# to the approximate ones, if they are 65536 or more. (lengths, query heads,
+# kv heads, head_dim, block, blocks per row, top_k): lines on a tile and inside
+# one, sequences that end before, on, one past and far past the line, exactly
+# 65536 queries and fewer.
+SPLITS = [([255 * 16 + 1], 18, 1, 64, 16, 256, 17), ([256 * 17], 17, 1, 64, 17, 256, 10),
+          ([3840], 18, 2, 64, 16, 300, 13), ([3841, 100, 3839, 3900, 1], 4, 2, 64, 16, 300, 13),
+          ([2048, 2049, 4096, 700], 8, 2, 128, 16, 256, 10), ([257 * 20], 26, 2, 128, 20, 257, 17),
+          ([3841, 3900], 2, 2, 64, 16, 256, 12)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("offset", [0.0, 3.0])
+@pytest.mark.parametrize("case", SPLITS)
+def test_gate_split_by_position_matches_oracle_and_general_path(device, case, offset, dtype):
+    lens, hq, hk, d, bs, n, k = case
+    cfg = MoBAConfig(block_size=bs, top_k=k, dtype=dtype)
+    g = torch.Generator().manual_seed(len(lens) + d)
+    q = torch.randn((1, sum(lens), hq, d), generator=g).to(dtype)
+    kbar = torch.randn((len(lens), hk, n, d), generator=g) * bs ** -0.5 + offset * torch.randn(
+        (1, hk, 1, d), generator=g)
+    kbar = kbar.to(dtype)
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    take, qd, kd, cud = k - 1, q.to(device), kbar.to(device), cu.to(device)
+    got = _gate(qd, kd, cfg, max(lens), take, cud)
+    assert torch.equal(got, _gate(_shifted(qd), kd, cfg, max(lens), take, cud))
+    need = -(-max(lens) // bs)  # the oracle's rows: what the longest sequence has
+    ref = c_oracle.gate_select(q, kbar[:, :, :need].contiguous(), oracle_cfg(cfg), cu, max(lens))
+    assert torch.equal(got.cpu(), ref)
