@@ -2,6 +2,7 @@
 `moba_backward_step`): the stages of `pooling`, `gating`, `routing`, `moba_fwd`
 and `moba_bwd` in order, without their per-stage allocations and calls."""
 
+import ctypes
 from dataclasses import dataclass
 
 import torch
@@ -10,13 +11,15 @@ from moba import _lib
 from moba.config import MoBAConfig
 from moba.kernels.routing import MAX_SEGMENTS, segment_entries
 
+_POINTERS = _lib.Step.q.offset  # the device addresses end the struct
+
 
 @dataclass(frozen=True)
 class SavedStep:
     """What a forward keeps for its backward: the call's shape and one buffer
     holding the CSC index, the (m, l) pairs and lse."""
 
-    shape: _lib.Step  # its pointers are not read again
+    shape: _lib.Step  # without addresses: the backward fills in its own
     saved: torch.Tensor
     cu_seqlens: torch.Tensor | None
 
@@ -44,7 +47,10 @@ def forward(q, k, v, cfg: MoBAConfig, causal: bool, cu_seqlens, max_seqlen, keep
     step.cu_seqlens = cu_seqlens.data_ptr() if packed else None
     step.out, step.saved, step.temp = out.data_ptr(), saved.data_ptr(), temp.data_ptr()
     _lib.run_step("moba_forward_step", step, _lib.stream_handle(dev))
-    return out, SavedStep(step, saved, cu_seqlens) if keep else None
+    if not keep:
+        return out, None
+    ctypes.memset(ctypes.byref(step, _POINTERS), 0, ctypes.sizeof(step) - _POINTERS)
+    return out, SavedStep(step, saved, cu_seqlens)
 
 
 def backward(dout, q, k, v, out, kept: SavedStep, dkv_dtype=None):
