@@ -728,18 +728,18 @@ static int set_lds(K kernel, size_t bytes) {
 
 }  // namespace moba
 
-extern "C" int moba_attend(const void* q, const void* k, const void* v,
-                           const int32_t* col_nnz, const int32_t* col_offsets,
-                           const int32_t* row_indices, const int32_t* head_indices,
-                           const int32_t* slot_of_pair, const int32_t* order,
-                           float* part_ml, void* part_acc,
-                           const int32_t* cu_seqlens, int64_t batch, int64_t seq_len,
-                           int64_t max_seqlen, int64_t h_q, int64_t h_kv,
-                           int64_t head_dim, int64_t n_blocks, int64_t block_size,
-                           int64_t slots, int64_t index_cap, int64_t index_stride,
-                           const int32_t* segments, const int32_t* seg_split,
-                           const int32_t* seg_counts, int64_t seg_cap,
-                           int causal, int dtype, int acc_dtype, void* stream) {
+int moba::attend(const void* q, const void* k, const void* v,
+                 const int32_t* col_nnz, const int32_t* col_offsets,
+                 const int32_t* row_indices, const int32_t* head_indices,
+                 const int32_t* slot_of_pair, const int32_t* order,
+                 float* part_ml, void* part_acc,
+                 const int32_t* cu_seqlens, int64_t batch, int64_t seq_len,
+                 int64_t max_seqlen, int64_t h_q, int64_t h_kv,
+                 int64_t head_dim, int64_t n_blocks, int64_t block_size,
+                 int64_t slots, int64_t index_cap, int64_t index_stride,
+                 const int32_t* segments, const int32_t* seg_split,
+                 const int32_t* seg_counts, int64_t seg_cap,
+                 int causal, int dtype, int acc_dtype, void* stream, bool cleared) {
   using namespace moba;
   AttnArgs a;
   Geometry g;
@@ -756,11 +756,13 @@ extern "C" int moba_attend(const void* q, const void* k, const void* v,
   // Unwritten slots must read as m = -inf: the marker combine and dq reduce
   // rely on. The (m, l) pairs are cleared whole; l / acc of such slots are
   // never read.
-  const int64_t n_m = (g.packed ? 1 : batch) * h_q * seq_len * slots * 2;
-  hipLaunchKernelGGL(fill_f32_kernel, dim3(static_cast<unsigned>(cdiv(n_m, 256) < 8192 ? cdiv(n_m, 256) : 8192)),
-                     dim3(256), 0, s, part_ml, n_m, -INFINITY);
-  st = check_launch("moba_attend (fill)");
-  if (st) return st;
+  if (!cleared) {
+    const int64_t n_m = (g.packed ? 1 : batch) * h_q * seq_len * slots * 2;
+    hipLaunchKernelGGL(fill_f32_kernel, dim3(static_cast<unsigned>(cdiv(n_m, 256) < 8192 ? cdiv(n_m, 256) : 8192)),
+                       dim3(256), 0, s, part_ml, n_m, -INFINITY);
+    st = check_launch("moba_attend (fill)");
+    if (st) return st;
+  }
   st = attend_mfma(a, dtype, acc_dtype, batch * h_kv, s);
   if (st == MOBA_ERR_UNSUPPORTED) st = attend_f32(a, dtype, acc_dtype, batch * h_kv, s);
   if (st != MOBA_ERR_UNSUPPORTED) return st;
@@ -799,6 +801,25 @@ extern "C" int moba_attend(const void* q, const void* k, const void* v,
       return go(attend_simple_kernel<T, A, true, 64>);
     });
   });
+}
+
+extern "C" int moba_attend(const void* q, const void* k, const void* v,
+                           const int32_t* col_nnz, const int32_t* col_offsets,
+                           const int32_t* row_indices, const int32_t* head_indices,
+                           const int32_t* slot_of_pair, const int32_t* order,
+                           float* part_ml, void* part_acc,
+                           const int32_t* cu_seqlens, int64_t batch, int64_t seq_len,
+                           int64_t max_seqlen, int64_t h_q, int64_t h_kv,
+                           int64_t head_dim, int64_t n_blocks, int64_t block_size,
+                           int64_t slots, int64_t index_cap, int64_t index_stride,
+                           const int32_t* segments, const int32_t* seg_split,
+                           const int32_t* seg_counts, int64_t seg_cap,
+                           int causal, int dtype, int acc_dtype, void* stream) {
+  return moba::attend(q, k, v, col_nnz, col_offsets, row_indices, head_indices, slot_of_pair,
+                      order, part_ml, part_acc, cu_seqlens, batch, seq_len, max_seqlen, h_q,
+                      h_kv, head_dim, n_blocks, block_size, slots, index_cap, index_stride,
+                      segments, seg_split, seg_counts, seg_cap, causal, dtype, acc_dtype,
+                      stream, false);
 }
 
 extern "C" int moba_combine(const float* part_ml, const void* part_acc,

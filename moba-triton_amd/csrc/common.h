@@ -137,6 +137,25 @@ int64_t gate_f64_rows(const void* q, const void* kbar, const Geometry& g, int ta
 int gate_f64(const void* q, const void* kbar, int32_t* out, const int32_t* cu, const Geometry& g,
              int64_t rows, int take, int cur, int dtype, hipStream_t st);
 
+// moba_csc_build that where it is short also sets clear[0, n_clear) (on 16
+// bytes; null: none) to -inf and says so in `cleared`, and moba_attend with
+// its (m, l) pairs already so where `cleared`.
+int csc_build(const int32_t* block_idx, int32_t* col_nnz, int32_t* col_offsets,
+              int32_t* row_indices, int32_t* head_indices, int32_t* slot_of_pair, int32_t* order,
+              const int32_t* cu_seqlens, int64_t batch, int64_t seq_len, int64_t max_seqlen,
+              int64_t h_q, int64_t h_kv, int64_t n_blocks, int64_t slots, int64_t index_stride,
+              int32_t* segments, int32_t* seg_split, int32_t* seg_counts, int64_t seg_cap,
+              int64_t seg_len, int64_t max_seg, void* workspace, size_t workspace_bytes,
+              void* stream, float* clear, int64_t n_clear, bool* cleared);
+int attend(const void* q, const void* k, const void* v, const int32_t* col_nnz,
+           const int32_t* col_offsets, const int32_t* row_indices, const int32_t* head_indices,
+           const int32_t* slot_of_pair, const int32_t* order, float* part_ml, void* part_acc,
+           const int32_t* cu_seqlens, int64_t batch, int64_t seq_len, int64_t max_seqlen,
+           int64_t h_q, int64_t h_kv, int64_t head_dim, int64_t n_blocks, int64_t block_size,
+           int64_t slots, int64_t index_cap, int64_t index_stride, const int32_t* segments,
+           const int32_t* seg_split, const int32_t* seg_counts, int64_t seg_cap, int causal,
+           int dtype, int acc_dtype, void* stream, bool cleared);
+
 // Device view of where a sequence lives. Padded: sequence r is batch row r,
 // tokens [r*S, r*S + S). Packed: tokens [cu[r], cu[r+1]).
 struct SeqSpan {

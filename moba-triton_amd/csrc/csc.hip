@@ -601,11 +601,34 @@ inline bool mid_takes(int64_t n_blocks, int64_t units) {
   return n_blocks <= kMidCols && units <= kMidUnits * (kMidCols / n_blocks);
 }
 
+// csc_mid_kernel leaves most of the chip idle, so workgroups added at its end clear
+// the attention stage's (m, l) pairs meanwhile, in place of a launch of their
+// own: forward [4, 1000, 16/4, 128], top_k 4, 93.1 -> 91.5 us a call, forward
+// and backward [1, 2048, 4, 64], top_k 8, 189 -> 186. On longer calls the
+// launch is nothing, and pairs cleared in the index build (beside the column
+// order) are out of the caches by the time attention writes them: [1, 32768,
+// 32/8, 128] 4753 -> 4870, eight packed sequences of 572K tokens 6001 -> 6030.
+// So there the attention stage clears them.
+//
+// This workgroup's share, of `parts`, of p[0, n) = -inf; p on 16 bytes.
+__device__ inline void clear_share(float* __restrict__ p, int64_t n, int64_t part, int64_t parts) {
+  const float4 v = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+  const int64_t stride = parts * blockDim.x;
+  const int64_t i0 = part * blockDim.x + threadIdx.x;
+  for (int64_t i = i0; i < n / 4; i += stride) reinterpret_cast<float4*>(p)[i] = v;
+  if (i0 < n % 4) p[n / 4 * 4 + i0] = -INFINITY;
+}
+
 __global__ void __launch_bounds__(1024)
 csc_mid_kernel(int32_t* __restrict__ table, int32_t* __restrict__ col_nnz,
                int32_t* __restrict__ col_offsets, int32_t* __restrict__ order, int nb, int units,
                int64_t seg_len, int max_seg, int32_t* __restrict__ seg, int32_t* __restrict__ split,
-               int32_t* __restrict__ counts, int64_t seg_cap) {
+               int32_t* __restrict__ counts, int64_t seg_cap, int64_t pairs,
+               float* __restrict__ clear, int64_t n_clear) {
+  if (blockIdx.x >= pairs) {
+    clear_share(clear, n_clear, blockIdx.x - pairs, gridDim.x - pairs);
+    return;
+  }
   __shared__ int32_t psum[1024];  // [parts][nb]: sums, then each part's base
   __shared__ int32_t nnz[1024], by_rank[1024];
   __shared__ int32_t wtot[16];
@@ -721,16 +744,16 @@ extern "C" size_t moba_csc_workspace_size(int64_t batch, int64_t rows_per_seq, i
   return det > cur ? det : cur;
 }
 
-extern "C" int moba_csc_build(const int32_t* block_idx, int32_t* col_nnz,
-                              int32_t* col_offsets, int32_t* row_indices,
-                              int32_t* head_indices, int32_t* slot_of_pair,
-                              int32_t* order, const int32_t* cu_seqlens, int64_t batch,
-                              int64_t seq_len, int64_t max_seqlen, int64_t h_q,
-                              int64_t h_kv, int64_t n_blocks, int64_t slots,
-                              int64_t index_stride, int32_t* segments, int32_t* seg_split,
-                              int32_t* seg_counts, int64_t seg_cap, int64_t seg_len,
-                              int64_t max_seg, void* workspace, size_t workspace_bytes,
-                              void* stream) {
+int moba::csc_build(const int32_t* block_idx, int32_t* col_nnz,
+                    int32_t* col_offsets, int32_t* row_indices,
+                    int32_t* head_indices, int32_t* slot_of_pair,
+                    int32_t* order, const int32_t* cu_seqlens, int64_t batch,
+                    int64_t seq_len, int64_t max_seqlen, int64_t h_q,
+                    int64_t h_kv, int64_t n_blocks, int64_t slots,
+                    int64_t index_stride, int32_t* segments, int32_t* seg_split,
+                    int32_t* seg_counts, int64_t seg_cap, int64_t seg_len,
+                    int64_t max_seg, void* workspace, size_t workspace_bytes,
+                    void* stream, float* clear, int64_t n_clear, bool* cleared) {
   using namespace moba;
   Geometry g;
   const int64_t rps = cu_seqlens ? max_seqlen : seq_len;
@@ -770,6 +793,7 @@ extern "C" int moba_csc_build(const int32_t* block_idx, int32_t* col_nnz,
   const int tv = static_cast<int>(visible_queries(batch, h_q, g.rows_per_seq));
   const bool mid = tiled && n_win == 1 && mid_takes(n_blocks, up.units);
   const unsigned rhk = static_cast<unsigned>(batch * h_kv);
+  if (cleared) *cleared = mid;
   dim3 grid(static_cast<unsigned>(cdiv(g.rows_per_seq * slots, 256)),
             static_cast<unsigned>(batch * h_q));
   dim3 tgrid(static_cast<unsigned>(up.tiles), static_cast<unsigned>(batch * h_q));
@@ -818,9 +842,13 @@ extern "C" int moba_csc_build(const int32_t* block_idx, int32_t* col_nnz,
                        nullptr, index_stride);
   }
   if (mid) {
-    hipLaunchKernelGGL(csc_mid_kernel, dim3(rhk), dim3(1024), 0, s, table, col_nnz, col_offsets, order,
-                       static_cast<int>(n_blocks), static_cast<int>(up.units), seg_len,
-                       static_cast<int>(max_seg), segments, seg_split, seg_counts, seg_cap);
+    // Two 16-byte stores per thread of the clearing workgroups, and at most
+    // 1024 workgroups, which then loop.
+    const int64_t clearing = !clear ? 0 : cdiv(n_clear, 8192) < 1024 ? cdiv(n_clear, 8192) : 1024;
+    hipLaunchKernelGGL(csc_mid_kernel, dim3(rhk + static_cast<unsigned>(clearing)), dim3(1024), 0, s,
+                       table, col_nnz, col_offsets, order, static_cast<int>(n_blocks),
+                       static_cast<int>(up.units), seg_len, static_cast<int>(max_seg), segments,
+                       seg_split, seg_counts, seg_cap, static_cast<int64_t>(rhk), clear, n_clear);
     window_place(0, n_blocks);
     return check_launch("moba_csc_build");
   }
@@ -857,4 +885,21 @@ extern "C" int moba_csc_build(const int32_t* block_idx, int32_t* col_nnz,
                        head_indices, slot_of_pair, index_stride);
   }
   return check_launch("moba_csc_build");
+}
+
+extern "C" int moba_csc_build(const int32_t* block_idx, int32_t* col_nnz,
+                              int32_t* col_offsets, int32_t* row_indices,
+                              int32_t* head_indices, int32_t* slot_of_pair,
+                              int32_t* order, const int32_t* cu_seqlens, int64_t batch,
+                              int64_t seq_len, int64_t max_seqlen, int64_t h_q,
+                              int64_t h_kv, int64_t n_blocks, int64_t slots,
+                              int64_t index_stride, int32_t* segments, int32_t* seg_split,
+                              int32_t* seg_counts, int64_t seg_cap, int64_t seg_len,
+                              int64_t max_seg, void* workspace, size_t workspace_bytes,
+                              void* stream) {
+  return moba::csc_build(block_idx, col_nnz, col_offsets, row_indices, head_indices,
+                         slot_of_pair, order, cu_seqlens, batch, seq_len, max_seqlen, h_q, h_kv,
+                         n_blocks, slots, index_stride, segments, seg_split, seg_counts,
+                         seg_cap, seg_len, max_seg, workspace, workspace_bytes, stream, nullptr,
+                         0, nullptr);
 }

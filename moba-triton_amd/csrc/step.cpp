@@ -180,15 +180,18 @@ extern "C" int moba_forward_step(moba_step* step, void* stream) {
                           s.head_dim, s.n_blocks, s.block_size, s.slots, s.take,
                           static_cast<int>(s.always_current), dt, t.gate_ws, h.gate_ws, stream));
   if (st) return st;
-  st = stage(3, moba_csc_build(t.ids, v.nnz, v.offsets, v.entries, v.entries + 1, v.entries + 2,
-                               v.order, cu, s.batch, s.seq_len, h.rps, s.h_q, s.h_kv, s.n_blocks,
-                               s.slots, 3, v.seg, v.split, v.counts, v.seg ? h.seg_cap : 0,
-                               s.seg_len > 0 ? s.seg_len : 1, s.max_seg, t.csc_ws, h.csc_ws, stream));
+  bool cleared = false;
+  st = stage(3, csc_build(t.ids, v.nnz, v.offsets, v.entries, v.entries + 1, v.entries + 2, v.order,
+                          cu, s.batch, s.seq_len, h.rps, s.h_q, s.h_kv, s.n_blocks, s.slots, 3,
+                          v.seg, v.split, v.counts, v.seg ? h.seg_cap : 0,
+                          s.seg_len > 0 ? s.seg_len : 1, s.max_seg, t.csc_ws, h.csc_ws, stream,
+                          v.ml, 2 * h.n, &cleared));
   if (st) return st;
-  st = stage(4, moba_attend(s.q, s.k, s.v, v.nnz, v.offsets, v.entries, v.entries + 1, v.entries + 2,
-                            v.order, v.ml, t.acc, cu, s.batch, s.seq_len, s.max_seqlen, s.h_q, s.h_kv,
-                            s.head_dim, s.n_blocks, s.block_size, s.slots, h.cap, 3, v.seg, v.split,
-                            v.counts, v.seg ? h.seg_cap : 0, static_cast<int>(s.causal), dt, dt, stream));
+  st = stage(4, attend(s.q, s.k, s.v, v.nnz, v.offsets, v.entries, v.entries + 1, v.entries + 2,
+                       v.order, v.ml, t.acc, cu, s.batch, s.seq_len, s.max_seqlen, s.h_q, s.h_kv,
+                       s.head_dim, s.n_blocks, s.block_size, s.slots, h.cap, 3, v.seg, v.split,
+                       v.counts, v.seg ? h.seg_cap : 0, static_cast<int>(s.causal), dt, dt, stream,
+                       cleared));
   if (st) return st;
   return stage(5, moba_combine(v.ml, t.acc, s.out, v.lse, s.packed ? 1 : s.batch, s.seq_len, s.h_q,
                                s.head_dim, s.slots, dt, dt, stream));

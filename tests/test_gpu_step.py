@@ -57,3 +57,26 @@ def test_step_errors_name_the_stage(device):
     for call in (lambda: build_csc_fused(q, k, cfg), lambda: moba_forward(q, k, v, cfg)):
         with pytest.raises(ValueError, match="moba_gate: gate supports at most 128"):
             call()
+
+
+# Where the (m, l) pairs are cleared: beside the one-launch middle of the index
+# build on short calls, by the attention stage on others (few and many columns,
+# one and several rows).
+@pytest.mark.parametrize("s,b,hq,hk,bs,k", [(515, 2, 4, 2, 64, 4), (20011, 1, 4, 2, 64, 5),
+                                            (9000, 3, 8, 1, 128, 3), (32 * 4099 + 3, 1, 1, 1, 32, 2)])
+def test_step_clears_unwritten_slots(device, s, b, hq, hk, bs, k):
+    """Memory that held finite values before: slots without a block are still
+    left out of the merge."""
+    cfg = MoBAConfig(block_size=bs, top_k=k, dtype=torch.bfloat16)
+    q, do = make_qkv((b, s, hq, 64), torch.bfloat16, seed=3, device=device, n=2)
+    kk, v = make_qkv((b, s, hk, 64), torch.bfloat16, seed=4, device=device, n=2)
+    index = build_csc_fused(q, kk, cfg)
+    results = []
+    for given in (index, None):
+        x = [z.clone().requires_grad_(True) for z in (q, kk, v)]
+        torch.cuda.empty_cache()
+        old = torch.full((b * s * hq * k * 80,), 3.0, device=device)
+        del old  # its block serves the next allocations
+        out = moba_attention(*x, cfg, index=given)
+        results.append((out.detach(), *torch.autograd.grad(out, x, do)))
+    assert all(torch.equal(a, c) for a, c in zip(*results))
