@@ -325,8 +325,10 @@ bwd_f32_kernel(AttnArgs a) {
   auto stage = [&](int par) {
     if (tid < NQ) {
       s_lim[tid] = c_lim;
-      s_lse[tid] = ld.x;
-      s_delta[tid] = ld.y;
+      // A dead entry has read the call's first row: with that row's delta
+      // NaN or infinite, 0 * (dP - delta) would reach every key's dK.
+      s_lse[tid] = c_dst < 0 ? INFINITY : ld.x;
+      s_delta[tid] = c_dst < 0 ? 0.f : ld.y;
       s_dst[par][tid] = c_dst;
     }
 #pragma unroll
