@@ -434,6 +434,11 @@ __device__ constexpr int bq_swz(int row) {
   return (((row >> 1) & 1) << 2) | ((row >> 1) & 2) | ((row >> 3) & 1);
 }
 
+// (lse, delta) of a column's dead entries (the last step's past its end):
+// they make P and dS zero. With those of any row of the call in their place,
+// exp2(0 - lse) may overflow the 16-bit P, and delta may be NaN.
+__device__ __attribute__((aligned(8))) float kDeadStats[2] = {INFINITY, 0.f};
+
 // dK, dV of this lane's key: register v of tile dt is feature f0 + 32dt +
 // 8(v/4) + v%4. A segment of a cut column leaves its float32 sums in its
 // scratch slot ([2][BS][D]: dK scaled, dV); the finishing pass adds the
@@ -578,7 +583,7 @@ bwd_mfma_kernel(AttnArgs a) {
   float n_lse = 0.f, n_dl = 0.f;
   auto fetch = [&]() {  // step g + 1: rows via s_qoff, lse / delta via n_pr
     if (idx_wave) {
-      const float2 ld = *reinterpret_cast<const float2*>(a.lse_delta + 2 * n_pr);
+      const float2 ld = *reinterpret_cast<const float2*>((n_dst < 0 ? kDeadStats : a.lse_delta) + 2 * n_pr);
       n_lse = ld.x;
       n_dl = ld.y;
     }
@@ -675,10 +680,10 @@ bwd_mfma_kernel(AttnArgs a) {
     __syncthreads();
     const int64_t* s_dst = s_dst_[par];
     // Every entry of the step sees the whole block (a strictly past, full
-    // block) or is dead: the causal masks can go. A dead entry's Q and dO
-    // rows are zero, so it adds nothing to dK / dV either way, and its dQ is
-    // never stored. Each wave reads the same NQ limits, so the vote is
-    // uniform over the workgroup.
+    // block) or is dead: the causal masks can go. A dead entry's rows are
+    // zero and kDeadStats makes its P and dS zero, so it adds nothing to
+    // dK / dV either way, and its dQ is never stored. Each wave reads the
+    // same NQ limits, so the vote is uniform over the workgroup.
     const bool all_visible = __all(lane >= NQ || s_lim[lane < NQ ? lane : 0] == BS - 1 ||
                                    s_lim[lane < NQ ? lane : 0] < 0);
     // Unconditional (past the column's end they read valid, clamped rows
@@ -963,7 +968,7 @@ bwd_wide_kernel(AttnArgs a) {
   float n_lse = 0.f, n_dl = 0.f;
   auto fetch_stats = [&]() {
     if (idx_wave) {
-      const float2 ld = *reinterpret_cast<const float2*>(a.lse_delta + 2 * n_pr);
+      const float2 ld = *reinterpret_cast<const float2*>((n_dst < 0 ? kDeadStats : a.lse_delta) + 2 * n_pr);
       n_lse = ld.x;
       n_dl = ld.y;
     }
