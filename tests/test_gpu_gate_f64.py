@@ -128,3 +128,37 @@ def test_gate_split_by_position_matches_oracle_and_general_path(device, case, of
     need = -(-max(lens) // bs)  # the oracle's rows: what the longest sequence has
     ref = c_oracle.gate_select(q, kbar[:, :, :need].contiguous(), oracle_cfg(cfg), cu, max(lens))
     assert torch.equal(got.cpu(), ref)
+
+
+def _off_by_one(t):
+    """The same float32 values 4 bytes off a 16-byte boundary: gate_exact_kernel."""
+    buf = torch.empty(t.numel() + 1, device=t.device, dtype=t.dtype)
+    buf[1:] = t.reshape(-1)
+    return buf[1:].view(t.shape)
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("kind", ["ties", "inf_nan", "tiny", "huge"])
+def test_gate_f64_float32_special_values_match_exact_path(device, kind, d):
+    """As above in float32: inf and NaN never rank, scores that round to 0 or
+    overflow tie. The ids of the exact kernel and of the oracle."""
+    cfg = MoBAConfig(block_size=16, top_k=5, dtype=torch.float32, always_select_current=kind != "ties")
+    lens = [700, 33, 1, 417]
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    g = torch.Generator().manual_seed(6)
+    q = torch.randn((1, sum(lens), 4, d), generator=g)
+    kbar = torch.randn((len(lens), 2, 44, d), generator=g)
+    if kind == "ties":
+        q, kbar = q.sign(), (kbar * 0.4).round()
+    elif kind == "inf_nan":
+        kbar[0, 0, 3, 5], kbar[0, 1, 7, 0], kbar[0, 0, 20, 1] = float("inf"), float("nan"), -float("inf")
+        q[0, 300, 1, 2], q[0, 500:, 2, 3] = float("nan"), -float("inf")
+    elif kind == "tiny":  # products of 1e-46 and below: most scores round to 0
+        q, kbar = q * 1e-23, kbar * 1e-23
+    else:  # of 1e40: most scores overflow
+        q, kbar = q * 1e20, kbar * 1e20
+    take, cud = cfg.past_blocks_selected(44), cu.to(device)
+    qd, kd = q.to(device), kbar.to(device)
+    got = _gate(qd, kd, cfg, max(lens), take, cud)
+    assert torch.equal(got, _gate(_off_by_one(qd), kd, cfg, max(lens), take, cud))
+    assert torch.equal(got.cpu(), c_oracle.gate_select(q, kbar, oracle_cfg(cfg), cu, max(lens)))
