@@ -645,7 +645,8 @@ bwd_mfma_kernel(AttnArgs a) {
   }
   if (c.n > 0) {
     c_lim = n_lim; c_dst = n_dst; c_lse = n_lse; c_dl = n_dl;
-    derive();  // s_qoff now describes step 1; every thread read step 0's above
+    __syncthreads();  // every thread has read step 0's s_qoff
+    derive();
   }
   // Stages one step: its limits, row statistics, dQ destinations (parity
   // par) and its Q / dO rows, row-major (the dV / dK products read them
