@@ -595,10 +595,14 @@ seg_build_kernel(const int32_t* __restrict__ col_nnz, const int32_t* __restrict_
 // launch of a few microseconds with little in it. [1, 2048, 4, 64], 128-key
 // blocks, top_k 8: the build's kernels 33 -> 20 us. kMidUnits bounds the
 // units a thread walks; beyond it the six kernels spread over more of the chip.
-constexpr int64_t kMidCols = 1024;
+// kMidCols bounds the columns a thread compares its own with, one by one: the
+// whole build, here and in the six kernels, at 128 columns 59 / 67 us, 256:
+// 62 / 67, 300: 68 / 71, 400: 45 / 45 and 39.8 / 37.8, 512: 71 / 70 and 44 /
+// 39, 700: 97 / 87, 1024: 102 / 80 (one or 32 heads, blocks of 16 to 128).
+constexpr int64_t kMidCols = 320;
 constexpr int64_t kMidUnits = 32;
 inline bool mid_takes(int64_t n_blocks, int64_t units) {
-  return n_blocks <= kMidCols && units <= kMidUnits * (kMidCols / n_blocks);
+  return n_blocks <= kMidCols && units <= kMidUnits * (1024 / n_blocks);
 }
 
 // csc_mid_kernel leaves most of the chip idle, so workgroups added at its end clear

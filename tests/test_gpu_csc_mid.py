@@ -14,12 +14,14 @@ pytestmark = pytest.mark.gpu
 
 # (lengths or S, batch, query heads, kv heads, columns, slots): one entry per
 # query (rows of ids in halves), queries that straddle rows of ids, one tile
-# and one column, the last column count taken (one part), the last unit count
-# taken and one more (the general build on both sides), packed sequences down
-# to one token.
+# and one column, far more columns than it takes (the general build on both
+# sides), the last unit count taken with 64-query units and one more, packed
+# sequences down to one token, the last column count taken, with the last unit
+# count and two more, and one more column.
 CASES = [(1000, 2, 4, 2, 16, 1), (777, 1, 6, 2, 7, 3), (9, 1, 1, 1, 1, 5), (2048, 1, 1, 1, 1024, 8),
          (64 * 32, 1, 4, 1, 256, 4), (64 * 32 + 1, 1, 4, 1, 256, 4), (600, 3, 3, 3, 33, 17),
-         ([300, 1, 64, 555, 2], 1, 4, 2, 20, 4), ([5, 40], 1, 8, 1, 3, 64)]
+         ([300, 1, 64, 555, 2], 1, 4, 2, 20, 4), ([5, 40], 1, 8, 1, 3, 64),
+         (48 * 64, 1, 2, 1, 320, 8), (48 * 64 + 1, 1, 2, 1, 320, 8), (3210, 1, 1, 1, 321, 8)]
 
 
 @pytest.mark.parametrize("entries", ["0", "24"])
