@@ -79,22 +79,45 @@ constexpr int kTileQ = 1024;
 typedef int32_t i32x3 __attribute__((ext_vector_type(3), aligned(4)));
 constexpr int kTileT = 256;
 
+// Columns and units of a (row, kv head) pair that csc_mid_kernel takes (its
+// comment says why).
+constexpr int64_t kMidCols = 320;
+constexpr int64_t kMidUnits = 32;
+inline bool mid_takes(int64_t n_blocks, int64_t units) {
+  return n_blocks > 0 && n_blocks <= kMidCols && units <= kMidUnits * (1024 / n_blocks);
+}
+
 // Queries per tile (a *unit* of the deterministic build is one tile of one
 // query head): 1024, or 256 when 1024-query tiles would give fewer than 512
-// units, or 64 when 256-query tiles would. The scatter walks a unit's entries
-// in one serial chain, so a build with few units waits on that chain (256
-// units at [1,64K,4,64], 32 at [1,2K,4,64]); with more units, smaller tiles
-// cost more in count-table traffic (units x columns) than they save
-// (measured: 256 against 1024 at 64K 0.088 -> 0.072 ms, 128K no gain).
+// units, or 64 on short calls of those. The scatter walks a unit's entries in
+// one serial chain, so a build with few units waits on that chain (256 units
+// at [1,64K,4,64], 32 at [1,2K,4,64]); with more units, smaller tiles cost
+// more in count-table traffic (units x columns) than they save (measured: 256
+// against 1024 at 64K 0.088 -> 0.072 ms, 128K no gain).
+// 64 queries where 256 would give fewer than 512 units and csc_mid_kernel
+// takes the 64-query units ([1,2K,4,64], 128-key blocks: 22.4 us, with 256
+// queries 26.8). Failing that, 256 where it takes those and has few columns
+// (8K, 8 query / 2 kv heads, 128 columns: 32.1, with 64 queries 36.9; 300
+// columns 37.7 and 36.5). Failing that too, 64 while the table stays small, at
+// most 2^18 entries and 512 units of a pair: 1 head, 16K, 512 columns 35.6,
+// with 256 queries 38.5. Past those it loses: 1 head of 96K, 3072 columns, 86
+// against 74, of 64K, 512 columns, 45.9 against 41.4; 2 heads of one pair,
+// 25K, 200 columns (800 units) 39.5 against 38.7.
 // A query's ids count up to the last block its tile of visible_queries()
 // queries sees (256 or 1024, whatever the units are).
 inline int64_t visible_queries(int64_t batch, int64_t h_q, int64_t rows_per_seq) {
   const int64_t units = batch * h_q * ((rows_per_seq + kTileQ - 1) / kTileQ);
   return units < 512 ? 256 : kTileQ;
 }
-inline int64_t tile_queries(int64_t batch, int64_t h_q, int64_t rows_per_seq) {
+inline int64_t tile_queries(int64_t batch, int64_t h_q, int64_t h_kv, int64_t rows_per_seq,
+                            int64_t n_blocks) {
   const int64_t tq = visible_queries(batch, h_q, rows_per_seq);
-  return tq == 256 && batch * h_q * ((rows_per_seq + 255) / 256) < 512 ? 64 : tq;
+  const int64_t t64 = (rows_per_seq + 63) / 64, t256 = (rows_per_seq + 255) / 256;
+  if (tq != 256 || batch * h_q * t256 >= 512) return tq;
+  const int64_t group = h_kv > 0 ? h_q / h_kv : 1;
+  if (mid_takes(n_blocks, group * t64)) return 64;
+  if (n_blocks <= 256 && mid_takes(n_blocks, group * t256)) return 256;
+  return group * t64 <= 512 && batch * h_q * t64 * n_blocks <= 1 << 18 ? 64 : 256;
 }
 constexpr int kMaxBins = 16384;
 
@@ -599,11 +622,6 @@ seg_build_kernel(const int32_t* __restrict__ col_nnz, const int32_t* __restrict_
 // whole build, here and in the six kernels, at 128 columns 59 / 67 us, 256:
 // 62 / 67, 300: 68 / 71, 400: 45 / 45 and 39.8 / 37.8, 512: 71 / 70 and 44 /
 // 39, 700: 97 / 87, 1024: 102 / 80 (one or 32 heads, blocks of 16 to 128).
-constexpr int64_t kMidCols = 320;
-constexpr int64_t kMidUnits = 32;
-inline bool mid_takes(int64_t n_blocks, int64_t units) {
-  return n_blocks <= kMidCols && units <= kMidUnits * (1024 / n_blocks);
-}
 
 // csc_mid_kernel leaves most of the chip idle, so workgroups added at its end clear
 // the attention stage's (m, l) pairs meanwhile, in place of a launch of their
@@ -740,7 +758,8 @@ extern "C" size_t moba_csc_workspace_size(int64_t batch, int64_t rows_per_seq, i
   // Unit table and chunk sums of one column window. This is never smaller
   // than the atomic cursors of the untiled build (batch * h_kv * n_blocks),
   // which run in the same memory when the device lacks the LDS.
-  const UnitPlan p = unit_plan(rows_per_seq, h_q, h_kv, moba::tile_queries(batch, h_q, rows_per_seq));
+  const UnitPlan p = unit_plan(rows_per_seq, h_q, h_kv,
+                               moba::tile_queries(batch, h_q, h_kv, rows_per_seq, n_blocks));
   const int64_t width = n_blocks < moba::kDetMaxCols ? n_blocks : moba::kDetMaxCols;
   const size_t det = sizeof(int32_t) * static_cast<size_t>(batch * width *
                                                           (h_q * p.tiles + h_kv * p.nchunks));
@@ -792,7 +811,7 @@ int moba::csc_build(const int32_t* block_idx, int32_t* col_nnz,
   const size_t det_lds = 8 * static_cast<size_t>(win);
   const bool tiled = det_lds_ok(det_lds);
   const int64_t bs_eff = cdiv(g.rows_per_seq, n_blocks);
-  const int64_t tq = tile_queries(batch, h_q, g.rows_per_seq);
+  const int64_t tq = tile_queries(batch, h_q, h_kv, g.rows_per_seq, n_blocks);
   const UnitPlan up = unit_plan(g.rows_per_seq, h_q, h_kv, tq);
   const int tv = static_cast<int>(visible_queries(batch, h_q, g.rows_per_seq));
   const bool mid = tiled && n_win == 1 && mid_takes(n_blocks, up.units);

@@ -62,6 +62,14 @@ def test_workspace_queries_are_host_only():
     assert lib.moba_csc_workspace_size(1, 65536, 4, 4, 512, 8) == 4 * (4 * 256 + 4 * 16) * 512
     # 512K: 4 x 512 units at 1024 queries each. Chunk sums: 32 chunks of 16.
     assert lib.moba_csc_workspace_size(1, 524288, 4, 4, 4096, 8) == 4 * (4 * 512 + 4 * 32) * 4096
+    # 64-query units only where the short build takes them (16 columns, 32
+    # units of each of 4 pairs) or the table is small; one head over many
+    # columns keeps 256-query units (3072 columns x 384 units, chunks of 16).
+    assert lib.moba_csc_workspace_size(1, 2048, 4, 4, 16, 8) == 4 * (4 * 32 + 4 * 2) * 16
+    assert lib.moba_csc_workspace_size(1, 16384, 1, 1, 512, 8) == 4 * (256 + 16) * 512
+    assert lib.moba_csc_workspace_size(1, 98304, 1, 1, 3072, 8) == 4 * (384 + 24) * 3072
+    assert lib.moba_csc_workspace_size(1, 8192, 8, 2, 128, 8) == 4 * (8 * 32 + 2 * 8) * 128
+    assert lib.moba_csc_workspace_size(1, 128, 1, 0, 0, 8) == 0  # refused by the build itself
     # past 16384 columns: the table of one 16384-column window
     tiles = (1 << 22) // 1024
     chunk = -(-2 * tiles // 64)
