@@ -1066,9 +1066,9 @@ bwd_wide_kernel(AttnArgs a) {
     // Every entry sees the whole block or is dead: no causal masks.
     const int lim = s_lim[lane];
     const bool all_visible = __all(lim == BS - 1 || lim < 0);
-    // Unconditional (past the column's end clamped, valid rows). With four or
-    // more chunks per thread half of them wait until S and dP have left their
-    // registers.
+    // Unconditional (past the column's end clamped, valid rows). At 64 keys
+    // half of the chunks wait until S and dP have left their registers; at 32
+    // (8 chunks per thread, 1 wave per SIMD) there is room for all.
     constexpr int C0 = kTight ? CH / 2 : CH;
     fetch_stats();
     fetch_rows(0, C0);

@@ -603,8 +603,9 @@ seg_finish_kernel(AttnArgs a) {
   const int key_lim = static_cast<int>(c.key_end - c.key0);
   T* dK = static_cast<T*>(a.dk);
   T* dV = static_cast<T*>(a.dv);
-  // Thread -> (key, four features): D / 4 threads per key row (the MFMA
-  // backward, the only producer of segments, has D of 64 or 128).
+  // Thread -> (key, four features): D / 4 threads per key row (the 16-bit
+  // MFMA backward, whose segments these are, has D of 64 or 128; the float32
+  // one has a finishing pass of its own).
   const int v4 = static_cast<int>(a.D / 4);
   const int per = static_cast<int>(blockDim.x) / v4;
   const int c4 = static_cast<int>(threadIdx.x) % v4;

@@ -623,14 +623,16 @@ seg_build_kernel(const int32_t* __restrict__ col_nnz, const int32_t* __restrict_
 // 62 / 67, 300: 68 / 71, 400: 45 / 45 and 39.8 / 37.8, 512: 71 / 70 and 44 /
 // 39, 700: 97 / 87, 1024: 102 / 80 (one or 32 heads, blocks of 16 to 128).
 
-// csc_mid_kernel leaves most of the chip idle, so workgroups added at its end clear
-// the attention stage's (m, l) pairs meanwhile, in place of a launch of their
-// own: forward [4, 1000, 16/4, 128], top_k 4, 93.1 -> 91.5 us a call, forward
-// and backward [1, 2048, 4, 64], top_k 8, 189 -> 186. On longer calls the
-// launch is nothing, and pairs cleared in the index build (beside the column
-// order) are out of the caches by the time attention writes them: [1, 32768,
-// 32/8, 128] 4753 -> 4870, eight packed sequences of 572K tokens 6001 -> 6030.
-// So there the attention stage clears them.
+// csc_mid_kernel leaves most of the chip idle, so workgroups added at its end
+// clear the attention stage's (m, l) pairs meanwhile, in place of a launch of
+// their own. Whole calls with the pairs cleared here / by the attention stage,
+// us: forward [1, 2048, 4, 64] 52.7 / 55.5, [1, 8192, 4, 64] 76.6 / 78.1, 24
+// packed sequences of 54K tokens, 16/4 heads of 128, 855 / 861; and no loss
+// with many pairs: [1, 16384, 32/8, 128] (34 MB) 966 / 971, [1, 32768, 32/8,
+// 128] (67 MB) forward 1990 / 1996, forward and backward 4811 / 4820 (runs of
+// one side differ by 1.5%). Where the general kernels build the index the
+// attention stage clears them: cleared beside the column order instead, eight
+// packed sequences of 572K tokens took 6030 against 6001.
 //
 // This workgroup's share, of `parts`, of p[0, n) = -inf; p on 16 bytes.
 __device__ inline void clear_share(float* __restrict__ p, int64_t n, int64_t part, int64_t parts) {

@@ -290,15 +290,24 @@ int launch(const void* q, const void* kbar, int32_t* out, const int32_t* cu, con
 // float32 has no approximate kernel: 64K queries of 127 blocks take 33 us
 // (head_dim 64) and 54 us (128), and took 1330 and 2400 in gate_exact_kernel.
 //
-// With lists of 9 to 16 and more blocks than that, the line is drawn per
-// position instead of per call: the cost here grows with a query's past
-// blocks, the approximate kernels' hardly does. Measured over lists of 9 to 16
-// and both 16-bit types: 128K queries of 256 blocks 128 .. 294 us whole and
-// 116 .. 226 split (head_dim 64 and 128), 156K of 313 blocks 146 .. 347 and
-// 139 .. 287, 512K of 512 blocks 450 .. 1167 and 380 .. 1019. The two parts
-// run one after the other, so a split pays only where the first part fills
-// the chip by itself: 61K queries of it (512K of 2048 blocks) are even, 41K
-// (125K of 400, head_dim 128) lose 1% on some keys, 7K (8K of 256) 15 us.
+// With lists of 9 to 16 and 256 blocks or more, the line is drawn per position
+// instead of per call: the cost here grows with a query's past blocks, the
+// approximate kernels' hardly does. Against those kernels for the whole call,
+// over lists of 9 to 16 and both 16-bit types: 128K queries of 256 blocks 128
+// .. 294 us and 116 .. 226 split (head_dim 64 and 128), 156K of 313 blocks 146
+// .. 347 and 139 .. 287, 512K of 512 blocks 450 .. 1167 and 380 .. 1019. The
+// two parts run one after the other, so a split pays only where the first part
+// fills the chip by itself: 61K queries of it (512K of 2048 blocks) are even,
+// 41K (125K of 400, head_dim 128) lose 1% on some keys, 7K (8K of 256) 15 us.
+// Against this kernel for the whole call, top_k 10 .. 17, i.i.d. / offset
+// keys, whole and split: head_dim 128, 224 blocks 111 and 122 .. 140 / 151 ..
+// 228, 255 blocks 135 and 125 .. 142 / 152 .. 231; head_dim 64, 255 blocks 80
+// and 106 .. 114 / 120 .. 179. So below 256 nothing is split. The whole call
+// stays ahead for a while above it too (320 blocks: 190 against 156 .. 181 /
+// 241 .. 297 and 116 against 131 .. 146 / 195 .. 231; 512 blocks: 405 against
+// 254 .. 304 / 382 .. 488 and 254 against 211 .. 245 / 306 .. 427): the line
+// at 256 is on the safe side of where the two meet, about 300 blocks on i.i.d.
+// keys at head_dim 128 and 450 at 64.
 int64_t gate_f64_rows(const void* q, const void* kbar, const Geometry& g, int take, int dtype) {
   if ((g.head_dim != 64 && g.head_dim != 128) || take > 16 || g.rows * g.h_q > 65535) return 0;
   // Rows are read in 16-byte pieces.
