@@ -47,13 +47,15 @@ enum moba_status {
 
 enum moba_dtype { MOBA_BF16 = 0, MOBA_FP16 = 1, MOBA_FP32 = 2 };
 
-/* Library identity. moba_abi_version() is 6: (m, l) and (lse, delta) travel
+/* Library identity. moba_abi_version() is 7: (m, l) and (lse, delta) travel
  * as 8-byte pairs, the CSC index arrays take an element stride, the CSC
  * build can emit a segment list that attend and backward take, its
- * workspace is sized by rows per sequence, and moba_bwd takes the dK / dV
- * dtype (version 1 took separate statistics arrays; 2 had no index stride;
+ * workspace is sized by rows per sequence, moba_bwd takes the dK / dV dtype,
+ * and there are the moba_step calls (version 1 took separate statistics arrays; 2 had no index stride;
  * 3 no segments; 4 sized the CSC workspace by seq_len and ordered column
- * entries by atomic cursors; 5 wrote dK / dV in the input dtype only). */
+ * entries by atomic cursors; 5 wrote dK / dV in the input dtype only; 6 had
+ * no moba_step calls, cut no columns of float32 inputs in moba_bwd and sized
+ * the CSC workspace of short calls by larger tiles). */
 int moba_abi_version(void);
 const char* moba_last_error(void);
 const char* moba_status_string(int status);

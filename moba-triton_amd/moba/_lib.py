@@ -79,7 +79,7 @@ class LibraryMissing(RuntimeError):
 
 
 # Version of include/moba_hip.h these bindings follow.
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 
 def load() -> ctypes.CDLL:
@@ -95,14 +95,16 @@ def load() -> ctypes.CDLL:
         lib = ctypes.CDLL(str(LIB_PATH))
     except OSError as exc:
         raise LibraryMissing(f"cannot load {LIB_PATH}: {exc}") from exc
+    # The version first: a library of another one may lack entry points.
+    version = getattr(lib, "moba_abi_version", lambda: None)()
+    if version != ABI_VERSION:
+        raise LibraryMissing(
+            f"{LIB_PATH} has ABI version {version}, these bindings expect "
+            f"{ABI_VERSION}; rebuild it")
     for name, (res, args) in SIGNATURES.items():
         fn = getattr(lib, name)
         fn.restype = res
         fn.argtypes = args
-    if lib.moba_abi_version() != ABI_VERSION:
-        raise LibraryMissing(
-            f"{LIB_PATH} has ABI version {lib.moba_abi_version()}, these bindings expect "
-            f"{ABI_VERSION}; rebuild it")
     _lib = lib
     return lib
 

@@ -20,7 +20,21 @@ def declared_functions():
 
 def test_library_loads():
     lib = _lib.load()
-    assert lib.moba_abi_version() == 6
+    assert lib.moba_abi_version() == 7
+
+
+@pytest.mark.parametrize("version", [6, None])
+def test_library_of_another_version_is_refused_by_name(monkeypatch, version):
+    """Also where it lacks entry points that the bindings have."""
+    class Old:
+        pass
+
+    if version is not None:
+        Old.moba_abi_version = staticmethod(lambda: version)
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib.ctypes, "CDLL", lambda path: Old())
+    with pytest.raises(_lib.LibraryMissing, match="rebuild it"):
+        _lib.load()
 
 
 def test_every_declared_symbol_is_exported_and_bound():
