@@ -127,6 +127,13 @@ int make_geometry(Geometry* g, int64_t batch, int64_t seq_len,
                   int64_t head_dim, int64_t n_blocks, int64_t block_size,
                   int64_t slots, const int32_t* cu_seqlens);
 
+// Shapes of the attention stages' matrix kernels (attn_mfma.hip, attn_f32.hip).
+// Only those take a segment list; the FMA kernels run whole columns.
+constexpr bool matrix_shape(int64_t head_dim, int64_t block_size) {
+  return (head_dim == 64 || head_dim == 128) &&
+         (block_size == 32 || block_size == 64 || block_size == 128);
+}
+
 // Queries per tile of the approximate gate kernel.
 constexpr int kGateTile = 128;
 

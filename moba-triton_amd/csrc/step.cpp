@@ -113,8 +113,8 @@ BackTemp back_temp_of(const moba_step& s, const Shape& h) {
   t.lse_delta = c.take<float>(2 * h.rows);
   t.dq_part = c.take<char>(h.n * s.head_dim * h.esize);
   // Sums of cut columns' segments: float32, for float32 inputs float64 (two
-  // slots each).
-  t.scratch_cap = 2 * h.extra * (h.esize / 2);
+  // slots each); none where the kernels run whole columns.
+  t.scratch_cap = matrix_shape(s.head_dim, s.block_size) ? 2 * h.extra * (h.esize / 2) : 0;
   t.scratch = t.scratch_cap
                   ? c.take<float>(h.pairs * t.scratch_cap * 2 * s.block_size * s.head_dim)
                   : nullptr;

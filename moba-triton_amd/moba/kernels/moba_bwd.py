@@ -5,6 +5,7 @@ import torch
 from moba import _lib
 from moba.config import MoBAConfig
 from moba.gqa import head_group_size
+from moba.kernels.moba_fwd import has_matrix_kernel
 from moba.kernels.routing import CSCIndex, index_stride
 
 
@@ -61,9 +62,12 @@ def bwd_kernel(dout, q, k, v, lse_delta, cfg: MoBAConfig, index: CSCIndex, dk, d
     rows = index.col_nnz.shape[0]
     mx = index.max_seqlen if index.cu_seqlens is not None else s
     # float32 dK / dV sums of the segments of cut columns (float32 inputs:
-    # float64 sums, two float32 slots each)
-    scratch_cap, scratch = 0, None
-    if index.segments is not None and index.seg_cap > index.num_blocks:
+    # float64 sums, two float32 slots each); shapes without a matrix kernel
+    # run whole columns
+    segments, scratch_cap, scratch = index.segments, 0, None
+    if not has_matrix_kernel(d, cfg.block_size):
+        segments = None
+    if segments is not None and index.seg_cap > index.num_blocks:
         scratch_cap = 2 * (index.seg_cap - index.num_blocks) * (q.element_size() // 2)
         scratch = torch.empty(rows * h_kv * scratch_cap * 2 * cfg.block_size * d,
                               device=dev, dtype=torch.float32)
@@ -74,7 +78,7 @@ def bwd_kernel(dout, q, k, v, lse_delta, cfg: MoBAConfig, index: CSCIndex, dk, d
               _lib.ptr(index.order), _lib.ptr(dk), _lib.ptr(dv), _lib.ptr(dq_part),
               _lib.ptr(index.cu_seqlens), rows, s, mx, h_q, h_kv, d, index.num_blocks,
               cfg.block_size, index.max_slots, index.row_indices.shape[-1], index_stride(index),
-              _lib.ptr(index.segments), _lib.ptr(index.seg_split), _lib.ptr(index.seg_counts),
+              _lib.ptr(segments), _lib.ptr(index.seg_split), _lib.ptr(index.seg_counts),
               index.seg_cap, _lib.ptr(scratch), scratch_cap, int(bool(causal)),
               _lib.DTYPE_CODE[q.dtype], _lib.DTYPE_CODE[dq_part.dtype],
               _lib.DTYPE_CODE[dk.dtype], _lib.stream_handle(dev))

@@ -172,13 +172,18 @@ _LDS_BYTES = 160 * 1024
 MAX_HEAD_DIM = 1024
 
 
+def has_matrix_kernel(head_dim: int, block_size: int) -> bool:
+    """Whether attend and the backward have matrix kernels for the shape (of
+    contiguous aligned inputs); only those cut columns into segments."""
+    return head_dim in _MFMA_HEAD_DIMS and block_size in _MFMA_BLOCKS
+
+
 def fits_attend_lds(head_dim: int, block_size: int, dtype) -> tuple[bool, str]:
     """Whether the FMA attend kernel can run the shape (csrc/attn_simple.hip
     moba_attend): a group's 16 float32 query rows and score rows, plus at
     least one key row, within 160 KiB of LDS. Always true where the MFMA
     kernel takes the shape."""
-    if (dtype in (torch.bfloat16, torch.float16) and head_dim in _MFMA_HEAD_DIMS
-            and block_size in _MFMA_BLOCKS):
+    if dtype in (torch.bfloat16, torch.float16) and has_matrix_kernel(head_dim, block_size):
         return True, ""
     esize = torch.empty((), dtype=dtype).element_size()
     e = 16  # queries per group of the FMA kernel

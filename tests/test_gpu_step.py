@@ -6,6 +6,7 @@ import pytest
 import torch
 
 from conftest import make_qkv
+from moba import _lib
 from moba.config import MoBAConfig
 from moba.kernels.attention import moba_attention
 from moba.kernels.moba_fwd import moba_forward
@@ -80,3 +81,27 @@ def test_step_clears_unwritten_slots(device, s, b, hq, hk, bs, k):
         out = moba_attention(*x, cfg, index=given)
         results.append((out.detach(), *torch.autograd.grad(out, x, do)))
     assert all(torch.equal(a, c) for a, c in zip(*results))
+
+
+@pytest.mark.parametrize("d,bs,cuts", [(64, 64, True), (32, 64, False), (64, 16, False)])
+def test_segment_scratch_only_where_columns_are_cut(device, monkeypatch, d, bs, cuts):
+    """The stages called one by one: no scratch for segments at shapes whose
+    kernels run whole columns, and the same gradients as the step's."""
+    monkeypatch.setenv("MOBA_SEGMENT_ENTRIES", "64")
+    cfg = MoBAConfig(block_size=bs, top_k=3, dtype=torch.float32)
+    q, do = make_qkv((1, 700, 4, d), torch.float32, seed=5, device=device, n=2)
+    k, v = make_qkv((1, 700, 2, d), torch.float32, seed=6, device=device, n=2)
+    scratch, call = [], _lib.call
+
+    def spy(name, *args):
+        if name == "moba_bwd":
+            scratch.append(args[-7])  # scratch, scratch_cap, causal, three dtypes, stream
+        return call(name, *args)
+
+    monkeypatch.setattr(_lib, "call", spy)
+    grads = []
+    for index in (build_csc_fused(q, k, cfg), None):
+        x = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        grads.append(torch.autograd.grad(moba_attention(*x, cfg, index=index), x, do))
+    assert [s is not None for s in scratch] == [cuts]
+    assert all(torch.equal(a, b) for a, b in zip(*grads))

@@ -57,3 +57,23 @@ def test_null_buffers_are_refused():
         _lib.run_step("moba_forward_step", _step(), None)
     with pytest.raises(ValueError, match="kept nothing"):
         _lib.run_step("moba_backward_step", _step(keep=0), None)
+
+
+@pytest.mark.parametrize("dtype", [0, 2])
+@pytest.mark.parametrize("d,bs,cuts", [(64, 128, True), (128, 32, True), (256, 128, False), (64, 256, False)])
+def test_segment_scratch_only_where_columns_are_cut(d, bs, cuts, dtype):
+    """Scratch for the sums of cut columns' segments (2 block sums of dK and
+    dV per segment, float64 for float32 inputs) only at shapes whose kernels
+    cut columns."""
+    sizes = []
+    for seg_len in (0, 512):
+        a = _step(head_dim=d, block_size=bs, dtype=dtype, seg_len=seg_len)
+        _lib.run_step("moba_step_layout", a)
+        sizes.append(a.backward_temp)
+    if not cuts:
+        assert sizes[1] == sizes[0]
+        return
+    extra = 2 * 2048 * 8 // 512  # of each of 2 (row, kv head) pairs
+    scratch = 2 * 2 * extra * 2 * bs * d * (8 if dtype == 2 else 4)
+    assert sizes[0] < sizes[1]
+    assert sizes[1] >= 4 * 2048 * 8 * d * (4 if dtype == 2 else 2) + scratch
