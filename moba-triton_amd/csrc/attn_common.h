@@ -100,6 +100,21 @@ __device__ inline Column resolve_column(const AttnArgs& a, int64_t x, int64_t rh
   return c;
 }
 
+// Programs per pair, one of the call's n_cols (row, kv head) pairs, in a launch
+// of the matrix kernels; those past a pair's segment list do nothing.
+// Workgroups go to the 8 XCDs in turn, so with a multiple of 8 the longest
+// column of every pair, the first of its list, runs on the same XCD and the
+// shortest on another. So an odd number where the columns outnumber the 256
+// CUs: forward and backward [16, 1024, 4, 128], 128-key blocks, top_k 8, 446
+// -> 303 us, [8, 2048, 8/4, 64] 331 -> 297, and no loss over 80 shapes. With
+// fewer columns, each on a CU of its own, the odd number of programs puts two
+// on one more often than it balances XCDs ([1, 700, 16, 128], 64-key blocks,
+// top_k 3, 94 -> 102 us).
+inline unsigned column_programs(const AttnArgs& a, int64_t n_cols) {
+  if (!a.seg) return static_cast<unsigned>(a.n_blocks);
+  return static_cast<unsigned>(n_cols * a.n_blocks > 256 ? a.seg_cap | 1 : a.seg_cap);
+}
+
 // Token-major element offset of (query row value, head) for this column's row.
 __device__ inline int64_t q_offset(const AttnArgs& a, const Column& c, int32_t row, int32_t head) {
   const int64_t tok = a.cu ? row : c.r * a.S + row;

@@ -502,7 +502,7 @@ bool aligned(const AttnArgs& a) {
 
 template <int D, int BS>
 int launch_attend(const AttnArgs& a, int64_t n_cols, hipStream_t st) {
-  const dim3 grid(static_cast<unsigned>(a.seg ? a.seg_cap : a.n_blocks), static_cast<unsigned>(n_cols));
+  const dim3 grid(column_programs(a, n_cols), static_cast<unsigned>(n_cols));
   hipLaunchKernelGGL((attend_f32_kernel<D, BS>), grid, dim3(64 * fwd_waves(D, BS)), 0, st, a);
   return check_launch("moba_attend (float32)");
 }
@@ -516,7 +516,7 @@ int launch_bwd(const AttnArgs& args, int64_t n_cols, hipStream_t st) {
   if (a.seg && a.seg_cap > a.n_blocks &&
       (a.scratch_cap < 4 * (a.seg_cap - a.n_blocks) || (reinterpret_cast<uintptr_t>(a.seg_scratch) & 7)))
     a.seg = nullptr;
-  const dim3 grid(static_cast<unsigned>(a.seg ? a.seg_cap : a.n_blocks), static_cast<unsigned>(n_cols));
+  const dim3 grid(column_programs(a, n_cols), static_cast<unsigned>(n_cols));
   hipLaunchKernelGGL((bwd_f32_kernel<D, BS>), grid, dim3(4 * BS), 0, st, a);
   const int rc = check_launch("moba_bwd (float32)");
   if (rc || !a.seg || a.seg_cap == a.n_blocks) return rc;

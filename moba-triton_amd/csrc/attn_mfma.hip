@@ -376,7 +376,7 @@ attend_mfma_kernel(AttnArgs a) {
 
 template <typename T, typename A, int D, int BS>
 static int launch_attend(const AttnArgs& a, int64_t n_cols, hipStream_t st) {
-  dim3 grid(static_cast<unsigned>(a.seg ? a.seg_cap : a.n_blocks), static_cast<unsigned>(n_cols));
+  dim3 grid(column_programs(a, n_cols), static_cast<unsigned>(n_cols));
   hipLaunchKernelGGL((attend_mfma_kernel<T, A, D, BS>), grid, dim3(64 * attend_waves(D, BS)), 0, st, a);
   return check_launch("moba_attend (mfma)");
 }
@@ -1262,7 +1262,7 @@ bwd_wide_kernel(AttnArgs a) {
 
 template <typename T, typename A, int D, int BS>
 static int launch_bwd(const AttnArgs& a, int64_t n_cols, hipStream_t st) {
-  dim3 grid(static_cast<unsigned>(a.seg ? a.seg_cap : a.n_blocks), static_cast<unsigned>(n_cols));
+  dim3 grid(column_programs(a, n_cols), static_cast<unsigned>(n_cols));
   if constexpr (D == 128)
     hipLaunchKernelGGL((bwd_wide_kernel<T, A, BS>), grid, dim3(4 * BS), 0, st, a);
   else

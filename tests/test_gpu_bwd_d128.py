@@ -22,7 +22,9 @@ pytestmark = pytest.mark.gpu
 # (S or packed lengths, query heads, kv heads, block, top_k)
 CASES = [([63, 64, 65, 1, 129, 300], 1, 1, 32, 3), ([63, 64, 65, 1, 129, 300], 1, 1, 64, 2),
          ([63, 64, 65, 1, 129, 300], 1, 1, 128, 2), (513, 8, 2, 32, 5), (1000, 4, 1, 64, 4),
-         (777, 4, 4, 128, 3)]
+         (777, 4, 4, 128, 3),
+         # more than 256 columns: one program past every segment list
+         (2200, 2, 2, 32, 3)]
 
 
 def _inputs(case, dtype, device):

@@ -23,7 +23,9 @@ pytestmark = pytest.mark.gpu
 # (S or packed lengths, query heads, kv heads, head_dim, block, top_k)
 CASES = [(513, 4, 2, 64, 32, 5), (1000, 4, 4, 64, 64, 4), (777, 8, 2, 64, 128, 3),
          (300, 4, 1, 128, 32, 6), (449, 4, 2, 128, 64, 2), (900, 2, 2, 128, 128, 8),
-         ([200, 1, 33, 391], 4, 2, 64, 32, 3), ([64, 500, 129], 4, 4, 128, 128, 2)]
+         ([200, 1, 33, 391], 4, 2, 64, 32, 3), ([64, 500, 129], 4, 4, 128, 128, 2),
+         # more than 256 columns: one program past every segment list
+         (2200, 2, 2, 64, 32, 3)]
 
 
 def _inputs(case, device):
