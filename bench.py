@@ -82,6 +82,7 @@ def gate_flops(s, hq=HEADS, d=HEAD_DIM, bs=BLOCK):
 
 def _short_kernel(name):
     """`void moba::gate_mfma_kernel<...>(...)` -> `gate_mfma_kernel`."""
+    name = name.replace("(anonymous namespace)::", "")
     return name.split("<")[0].split("(")[0].replace("void ", "").split("::")[-1]
 
 
